@@ -1231,39 +1231,9 @@ write_back:
 }
 
 // ================================================================ kernels ==
-// Copies the launch arguments into LDS for the out-of-line exact path, one
-// dword per lane straight from the kernel argument segment (a reference to
-// the by-value argument would give every lane a private copy in scratch).
-// Thread-0 copy of the kernel arguments into LDS; uniform addresses, so the
-// reads are scalar loads of the kernarg segment (no private copy of the
-// by-value argument).
-__device__ __forceinline__ void stash_args(SampleArgs* dst) {
-    const uint32_t* src = (const uint32_t*)__builtin_amdgcn_kernarg_segment_ptr();
-    uint32_t* d = reinterpret_cast<uint32_t*>(dst);
-#pragma unroll
-    for (uint32_t i = 0; i < sizeof(SampleArgs) / 4; ++i) d[i] = src[i];
-}
-// As above, from the kernel's SampleArgs parameter wherever it lies in the
-// kernel arguments.
-__device__ __forceinline__ void stash_args(SampleArgs* dst, const SampleArgs& src) {
-    const uint32_t* s = reinterpret_cast<const uint32_t*>(&src);
-    uint32_t* d = reinterpret_cast<uint32_t*>(dst);
-#pragma unroll
-    for (uint32_t i = 0; i < sizeof(SampleArgs) / 4; ++i) d[i] = s[i];
-}
-// The kernel arguments thread 0 staged in LDS, read back as wave-uniform values.
-__device__ __forceinline__ SampleArgs uniform_args(const SampleArgs& s) {
-    constexpr uint32_t N = sizeof(SampleArgs) / 4;
-    static_assert(sizeof(SampleArgs) % 4 == 0, "args size");
-    uint32_t w[N];
-    const uint32_t* src = reinterpret_cast<const uint32_t*>(&s);
-#pragma unroll
-    for (uint32_t i = 0; i < N; ++i) w[i] = (uint32_t)__builtin_amdgcn_readfirstlane((int)src[i]);
-    SampleArgs r;
-    __builtin_memcpy(&r, w, sizeof(r));
-    return r;
-}
-// Parallel copy of the kernel's SampleArgs parameter into LDS (two dwords per
+// Copies the launch arguments into LDS for the out-of-line exact path (a
+// reference to the by-value argument would give every lane a private copy in
+// scratch). Parallel copy of the kernel's SampleArgs parameter into LDS (two dwords per
 // lane of the first wave), then a barrier: `src` is the kernel parameter
 // itself, read where it lies in the kernel arguments.
 __device__ __forceinline__ void stage_args(SampleArgs* dst, const SampleArgs& src) {

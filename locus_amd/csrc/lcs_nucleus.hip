@@ -33,9 +33,9 @@
 //
 // Bin-level decisions carry a 1e-10 relative guard (a target that close to
 // a bin or sub-bin edge takes both neighbours). A plan that would compact
-// more than kNucList candidates, or a decisive sub-bin group larger than the
-// kGroupMax (256) the workgroup ranks at once, resolves the row with the
-// exact single-workgroup path.
+// more than kNucList candidates resolves the row with the exact
+// single-workgroup path; a decisive sub-bin group larger than the kGroupMax
+// (256) the workgroup ranks at once (tied values) is first narrowed by key.
 #include <hip/hip_runtime.h>
 #include <math.h>
 #include <stdint.h>
@@ -53,7 +53,7 @@ constexpr int NT = kSliceThreads;
 constexpr int kNW = NT / kWave;
 constexpr uint32_t kNone = 0xffffffffu;
 constexpr uint32_t kNucCand = 128;     // top-n candidates one slice holds
-constexpr uint32_t kGroupMax = 4 * kWave;  // candidates one decisive group may hold
+constexpr uint32_t kGroupMax = 4 * kWave;  // candidates of a decisive group ranked at once
 constexpr uint32_t kNucKeyCache = 2048;     // compacted candidates the select finalize keeps in LDS
 constexpr float kL2E = 1.4426950408889634f;
 constexpr double kGuard = 1e-10;
@@ -78,6 +78,8 @@ struct NucLocal {
     uint32_t ngc[2];           // group sizes of alternate gathers (each reset one gather ahead)
     uint32_t fp_pos;           // first_prefix's position and prefix mass
     double fp_m;
+    uint32_t lg_n, lg_cb;      // nuc_large_group: candidates left, and the count and weight before them
+    double lg_mb;
     uint32_t out_flag;
     // the row state pass B's workgroups derive from pass A's records
     float st_maxl, st_sx;
@@ -1026,18 +1028,127 @@ __global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(1, 2))) void
 }
 
 // ========================================================= C: nuc_select ==
-// The select pass's row finalize: exact decisions over the compacted ranges.
-// Every thread of the workgroup calls it, with the kernel arguments staged
-// in g_nuc.l.args; out of line so that its live values do not crowd the
-// compaction pass.
-template <int G>
-__device__ __attribute__((noinline)) void nuc_select_fin(uint32_t row, bool exact) {
+// What a decision looks for in its group: the first position i >= pos, or
+// whose inclusive prefix weight P has (before + P) / norm >= reach (monotone
+// in i).
+struct NucTarget {
+    uint32_t pos;
+    double before, norm, reach;
+};
+// A decisive group larger than kGroupMax (the candidates with codes c0..c1):
+// narrowed to the at most kGroupMax candidates around its target, which are
+// ranked into gsorted with their weights in gw as the select finalize's gather
+// leaves a small group. Returns how many, with the group's candidates and
+// weight before them in lg_cb and lg_mb, or kNone when the row has to take the
+// exact path. Each step counts the keys left and sums their weights in up to
+// 256 buckets of equal width between the least and the greatest key, and keeps
+// the buckets where the target is first met (both neighbours when it lies
+// within the sums' rounding; the last bucket when nowhere). A rank key is the
+// value, then the id, so the same step separates distinct values and then the
+// ids of one value: bf16 logits tie by the hundred (151936 normal logits:
+// ~260 a value at a top-p cut), and a group of one value needs one step. 24
+// mixed bf16 rows, whose top-p rows took the exact path for such a group:
+// nuc_select_fin_kernel 1090 -> 26 us, the call 1122 -> 73 us. Out of line:
+// inlined at the three decisions it cost a call without a large group (32
+// masked rows) 0.6 of 42.7 us.
+__device__ __attribute__((noinline)) uint32_t nuc_large_group(uint32_t c0, uint32_t c1, uint32_t n,
+                                                              const uint64_t* list, float maxl, float inv_t,
+                                                              NucTarget tgt) {
     NucSmem& sm = g_nuc;
-    if (exact) {
-        exact_row<kSliceThreads, kFbBins, kFbCap, kFbHistCap, G>(sm.l.args, row, sm.u.ex);
-        return;
+    const uint32_t tid = tid_x();
+    const int lane = lane_id(), wv = (int)(tid / kWave);
+    uint32_t* bc = reinterpret_cast<uint32_t*>(sm.u.fc.gsorted);   // (both free: the group is not ranked yet)
+    double* bm = sm.u.fc.gw;
+    static_assert(kGroupMax == NT && kNW == 4, "one bucket and one group candidate per thread");
+    uint64_t glo = 0ull, ghi = ~0ull;   // the keys left
+    uint32_t cb = 0u, m = kNone;
+    double mb = 0.0;
+    auto each = [&](auto body) {
+        for (uint32_t i = tid; i < n; i += NT) {
+            const uint32_t c = g_code[i];
+            if (c >= c0 && c <= c1) {
+                const uint64_t key = i < kNucKeyCache ? g_nuc.u.fc.lkey[i] : list[i];
+                if (key >= glo && key <= ghi) body(key);
+            }
+        }
+    };
+    // (each step cuts the keys' range by 2^7 or more, unless the target meets
+    // the gap between two clusters of keys within the sums' rounding)
+    for (int it = 0; it < 10 && m > kGroupMax; ++it) {
+        bc[tid] = 0u;
+        bm[tid] = 0.0;
+        uint64_t kmin = ~0ull, nmax = ~0ull;
+        each([&](uint64_t key) {
+            kmin = u64_min(kmin, key);
+            nmax = u64_min(nmax, ~key);
+        });
+        kmin = block_min_u64<NT>(kmin, sm.l.ck);
+        const uint64_t kmax = ~block_min_u64<NT>(nmax, sm.l.ck);
+        const int bits = 64 - __builtin_clzll((kmax - kmin) | 1ull);
+        const int sh = bits > 8 ? bits - 8 : 0;
+        each([&](uint64_t key) {
+            const uint32_t b = (uint32_t)((key - kmin) >> sh);
+            atomicAdd(&bc[b], 1u);
+            atomicAdd(&bm[b], exp_f64((double)tempered(rank_val(key), maxl, inv_t)));
+        });
+        __syncthreads();
+        // inclusive prefix sums over the buckets (bucket tid)
+        const uint32_t cl = bc[tid];
+        const double ml = bm[tid];
+        uint32_t ci = wave_scan_incl_u(cl);
+        double mi = wave_scan_incl(ml);
+        if (lane == kWave - 1) { sm.l.nall[wv] = ci; sm.l.sraw[wv] = mi; }
+        __syncthreads();
+        double mt = 0.0;
+#pragma unroll
+        for (int w = 0; w < kNW; ++w) {
+            if (w < wv) { ci += sm.l.nall[w]; mi += sm.l.sraw[w]; }
+            mt += sm.l.sraw[w];
+        }
+        // (the sums' rounding: at most n 2^-53 of the weight left, n <= kNucList)
+        const double ge = 0x1p-37 * mt;
+        auto met = [&](double p) { return (cb + ci - 1u >= tgt.pos) || (tgt.before + p) / tgt.norm >= tgt.reach; };
+        const uint64_t h0 = ballot(met(mb + mi + ge)), h1 = ballot(met(mb + mi - ge));
+        if (lane == 0) {
+            sm.l.ipen[wv] = h0 ? (uint32_t)wv * kWave + (uint32_t)__builtin_ctzll(h0) : kNone;
+            sm.l.imsk[wv] = h1 ? (uint32_t)wv * kWave + (uint32_t)__builtin_ctzll(h1) : kNone;
+        }
+        __syncthreads();
+        const uint32_t lastb = (uint32_t)((kmax - kmin) >> sh);
+        uint32_t b0 = lastb, b1 = lastb;
+#pragma unroll
+        for (int w = 0; w < kNW; ++w) { b0 = min(b0, sm.l.ipen[w]); b1 = min(b1, sm.l.imsk[w]); }
+        if (tid == b0) { sm.l.lg_cb = cb + ci - cl; sm.l.lg_mb = mb + mi - ml; }
+        if (tid == b1) sm.l.lg_n = cb + ci;
+        __syncthreads();
+        cb = sm.l.lg_cb;
+        mb = sm.l.lg_mb;
+        m = sm.l.lg_n - cb;
+        glo = kmin + ((uint64_t)b0 << sh);
+        ghi = b1 >= lastb ? kmax : kmin + (((uint64_t)b1 + 1u) << sh) - 1u;
     }
-    const SampleArgs a = uniform_args(sm.l.args);
+    if (m > kGroupMax) return kNone;
+    if (tid == 0) sm.l.lg_n = 0u;
+    __syncthreads();   // (the buckets are read, lg_n is cleared)
+    each([&](uint64_t key) { g_nuc.u.fc.gkey[atomicAdd(&g_nuc.l.lg_n, 1u)] = key; });
+    __syncthreads();
+    if (tid < m) {
+        const uint64_t x = sm.u.fc.gkey[tid];
+        uint32_t rank = 0;
+        for (uint32_t j = 0; j < m; ++j) rank += sm.u.fc.gkey[j] < x ? 1u : 0u;
+        sm.u.fc.gsorted[rank] = x;
+        sm.u.fc.gw[rank] = exp_f64((double)tempered(rank_val(x), maxl, inv_t));
+    }
+    __syncthreads();
+    return m;
+}
+
+// The select pass's row finalize: exact decisions over the compacted ranges.
+// Every thread of the workgroup calls it. Returns true (uniformly) when the
+// row has to take the exact path.
+template <int G>
+__device__ __forceinline__ bool nuc_select_fin(const SampleArgs& a, uint32_t row) {
+    NucSmem& sm = g_nuc;
     const uint32_t tid = tid_x();
     const int lane = lane_id(), wv = (int)(tid / kWave);
     const lcs_params P = scalar_load(a.params + row);
@@ -1306,6 +1417,40 @@ __device__ __attribute__((noinline)) void nuc_select_fin(uint32_t row, bool exac
         return g_nuc.l.fp_pos;
     };
 
+    // The decision inside range k's sub-bins [s0, s1]: the first position i
+    // (of ng, in rank order) whose inclusive prefix weight P satisfies
+    // hit(i, P), with P and the candidate's key; kNone when there is none, and
+    // then ng is kNone when the group could not be narrowed. tgt: hit without
+    // what is not monotone in i, for the narrowing of a large group.
+    auto first_of_group = [&](uint32_t k, uint32_t s0, uint32_t s1, auto hit, const NucTarget& tgt, uint32_t& ng,
+                              double& p_at, uint64_t& key) -> uint32_t {
+        ng = gather(k, s0, s1);
+        uint32_t m = ng, gcb = 0u;
+        double gmb = 0.0;
+        if (ng > kGroupMax) {   // (uniform)
+            // a row whose penalty window is above the context's max_hist
+            // goes to the exact path, which reports it
+            const bool pen = penalties_active(P) && a.hist_off != nullptr;
+            const uint32_t hn = pen ? a.hist_off[row + 1] - a.hist_off[row] : 0u;
+            if (min(hn, P.repeat_last_n) > a.max_hist) {
+                ng = kNone;
+                return kNone;
+            }
+            m = nuc_large_group(k * kNucSub + s0, k * kNucSub + s1, n, list, maxl, inv_t, tgt);
+            if (m == kNone) {
+                ng = kNone;
+                return kNone;
+            }
+            gcb = g_nuc.l.lg_cb;
+            gmb = g_nuc.l.lg_mb;
+        }
+        const uint32_t pos = first_prefix(m, [&](uint32_t i, double pi) { return hit(gcb + i, gmb + pi); }, p_at);
+        if (pos == kNone) return kNone;
+        p_at += gmb;
+        key = g_nuc.u.fc.gsorted[pos];
+        return gcb + pos;
+    };
+
     NPROF(row, 10);
     // ---- decisions; `fail` sends the row to the exact path ----
     bool fail = sm.l.out_flag != 0u;
@@ -1324,15 +1469,17 @@ __device__ __attribute__((noinline)) void nuc_select_fin(uint32_t row, bool exac
         if (!find_count(K, kk, sk)) {
             fail = true;
         } else {
-            const uint32_t ng = gather(kk, sk, sk);
             const uint32_t pos = K - 1u - c_before(kk, sk);
-            if (ng > kGroupMax || pos >= ng) {
+            uint32_t ng;
+            double pm = 0.0;
+            uint64_t key = ~0ull;
+            const uint32_t at = first_of_group(kk, sk, sk, [&](uint32_t i, double) { return i == pos; },
+                                               NucTarget{pos, 0.0, 1.0, __builtin_huge_val()}, ng, pm, key);
+            if (at == kNone) {
                 fail = true;
             } else {
-                double pm = 0.0;
-                (void)first_prefix(ng, [&](uint32_t i, double) { return i == pos; }, pm);
                 SK = m_before(kk, sk) + pm;
-                key_k = sm.u.fc.gsorted[pos];
+                key_k = key;
             }
         }
     }
@@ -1349,21 +1496,19 @@ __device__ __attribute__((noinline)) void nuc_select_fin(uint32_t row, bool exac
         if (!f0 || !f1 || k0 != k1) {
             fail = true;
         } else {
-            const uint32_t ng = gather(k0, s0, s1);
-            if (ng > kGroupMax) {
+            // cum = (mass before the group + prefix) / S reaches top_p
+            const double mb0 = m_before(k0, s0);
+            uint32_t ng;
+            double pm = 0.0;
+            uint64_t key = ~0ull;
+            const uint32_t pos = first_of_group(k0, s0, s1, [&](uint32_t, double pi) { return (mb0 + pi) / SK >= tp; },
+                                                NucTarget{kNone, mb0, SK, tp}, ng, pm, key);
+            if (pos == kNone || c_before(k0, s0) + pos + 1u > K) {
                 fail = true;
             } else {
-                // cum = (mass before the group + prefix) / S reaches top_p
-                const double mb0 = m_before(k0, s0);
-                double pm = 0.0;
-                const uint32_t pos = first_prefix(ng, [&](uint32_t, double pi) { return (mb0 + pi) / SK >= tp; }, pm);
-                if (pos == kNone || c_before(k0, s0) + pos + 1u > K) {
-                    fail = true;
-                } else {
-                    keep_p = c_before(k0, s0) + pos + 1u;
-                    mass_p = mb0 + pm;
-                    key_p = sm.u.fc.gsorted[pos];
-                }
+                keep_p = c_before(k0, s0) + pos + 1u;
+                mass_p = mb0 + pm;
+                key_p = key;
             }
         }
     }
@@ -1433,31 +1578,29 @@ __device__ __attribute__((noinline)) void nuc_select_fin(uint32_t row, bool exac
             fail = true;
         } else {
             if (!f1) { k1 = k0; s1 = kNucSub - 1; }
-            const uint32_t ng = gather(k0, s0, s1);
-            if (ng > kGroupMax) {
-                fail = true;
-            } else {
-                // the first kept position whose prefix reaches r
-                const double r = r0 - m_before(k0, s0);
-                const uint32_t cb0 = c_before(k0, s0);
-                double pm = 0.0;
-                const uint32_t pos = first_prefix(ng, [&](uint32_t i, double pi) { return cb0 + i < keep && r - pi <= 0.0; }, pm);
-                if (pos != kNone) {
-                    chosen = (int32_t)rank_idx(sm.u.fc.gsorted[pos]);
-                } else if (last_key != ~0ull && cb0 + ng >= keep) {
-                    // ran past the group: the reference's fallback is the last
-                    // kept candidate, known when a cut produced `keep`
-                    chosen = (int32_t)rank_idx(last_key);
-                }
-                if (chosen < 0) fail = true;
+            // the first kept position whose prefix reaches r
+            const double r = r0 - m_before(k0, s0);
+            const uint32_t cb0 = c_before(k0, s0);
+            uint32_t ng;
+            double pm = 0.0;
+            uint64_t key = ~0ull;
+            const uint32_t pos = first_of_group(
+                k0, s0, s1, [&](uint32_t i, double pi) { return cb0 + i < keep && r - pi <= 0.0; },
+                NucTarget{kNone, 0.0, 1.0, r}, ng, pm, key);
+            if (pos != kNone) {
+                chosen = (int32_t)rank_idx(key);
+            } else if (ng != kNone && last_key != ~0ull && cb0 + ng >= keep) {
+                // ran past the group: the reference's fallback is the last
+                // kept candidate, known when a cut produced `keep`
+                chosen = (int32_t)rank_idx(last_key);
             }
+            if (chosen < 0) fail = true;
         }
     }
     NPROF(row, 14);
-    if (fail) {
-        // every thread agrees (all decisions above are block-uniform)
-        exact_row<kSliceThreads, kFbBins, kFbCap, kFbHistCap, G>(sm.l.args, row, sm.u.ex);
-        return;
+    if (fail) {   // every thread agrees (all decisions above are block-uniform)
+        __syncthreads();   // (the exact path reuses the LDS that they read)
+        return true;
     }
     if (tid == 0) {
         a.ids[row] = chosen;
@@ -1481,6 +1624,7 @@ __device__ __attribute__((noinline)) void nuc_select_fin(uint32_t row, bool exac
         }
     }
     NPROF(row, 16);
+    return false;
 }
 
 
@@ -1657,9 +1801,10 @@ __global__ __launch_bounds__(NT) void nuc_select_fin_kernel(SampleArgs a) {
     if (!nuc_fin_row(a, row, P, masked)) return;
     NPROF(row, 15);
     const bool exact = (a.nrow[row - a.nuc_row0].flags & kNucFallback) != 0u;
-    if (tid_x() == 0) stash_args(&sm.l.args, a);
-    __syncthreads();
-    nuc_select_fin<G>(row, exact);
+    if (exact || nuc_select_fin<G>(a, row)) {
+        stage_args(&sm.l.args, a);
+        exact_row<kSliceThreads, kFbBins, kFbCap, kFbHistCap, G>(sm.l.args, row, sm.u.ex);
+    }
 }
 
 // Host launchers: per chunk of kNucRows rows, three slice-parallel passes,
