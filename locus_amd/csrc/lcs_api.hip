@@ -23,8 +23,8 @@ hipError_t launch_general(const SampleArgs& a, hipStream_t st);
 hipError_t launch_nucleus(const SampleArgs& a, hipStream_t st);
 hipError_t launch_verify(const VerifyArgs& a, hipStream_t st);
 hipError_t launch_draft(const DraftArgs& a, hipStream_t st);
-hipError_t launch_lmhead(const LmArgs& a, hipStream_t st);
-uint32_t lmhead_cols(uint32_t vocab, uint32_t cus);
+hipError_t launch_lmhead(const LmArgs& a, uint32_t cus, hipStream_t st);
+uint32_t lmhead_max_blocks(uint32_t vocab, uint32_t cus);
 }  // namespace lcs
 
 struct lcs_ctx {
@@ -37,8 +37,8 @@ struct lcs_ctx {
     float* d_raw = nullptr;
     float* d_pen = nullptr;
     uint32_t* status = nullptr;
-    lcs::LmRec* lmrecs = nullptr;   // lm-head epilogue records: max_rows x blocks of >= kLmColsMin columns
-    uint32_t cus = 0;               // compute units of the device (the lm-head's block shape)
+    lcs::LmRec* lmrecs = nullptr;   // lm-head epilogue records: max_rows x lmhead_max_blocks
+    uint32_t cus = 256;             // compute units of the device (the lm-head's tile shape)
     // nucleus path workspace (kNucRows rows at a time)
     lcs::NucRow* nrow = nullptr;
     uint64_t* nh_pk = nullptr;
@@ -145,6 +145,8 @@ lcs_ctx* lcs_create(int device, uint32_t max_rows, uint32_t max_vocab, uint32_t 
     const size_t d_elems = (size_t)max_rows * c->max_hist;
     const size_t nuc_rows = max_rows < lcs::kNucRows ? max_rows : lcs::kNucRows;
     const size_t nh_elems = nuc_rows * lcs::kMaxSlices * lcs::kNucBins;
+    // (a smaller vocabulary than max_vocab never takes more blocks)
+    const size_t lm_blocks = lcs::lmhead_max_blocks(max_vocab, c->cus);
     hipError_t e = hipSuccess;
     if ((e = hipMalloc(&c->recs, rec_bytes)) != hipSuccess ||
         (e = hipMalloc(&c->srecs, srec_bytes)) != hipSuccess ||
@@ -152,8 +154,7 @@ lcs_ctx* lcs_create(int device, uint32_t max_rows, uint32_t max_vocab, uint32_t 
         (e = hipMalloc(&c->d_raw, d_elems * 4)) != hipSuccess ||
         (e = hipMalloc(&c->d_pen, d_elems * 4)) != hipSuccess ||
         (e = hipMalloc(&c->status, 4)) != hipSuccess ||
-        (e = hipMalloc(&c->lmrecs, (size_t)max_rows * ((max_vocab + lcs::kLmColsMin - 1) / lcs::kLmColsMin) *
-                                       sizeof(lcs::LmRec))) != hipSuccess ||
+        (e = hipMalloc(&c->lmrecs, (size_t)max_rows * lm_blocks * sizeof(lcs::LmRec))) != hipSuccess ||
         (e = hipMalloc(&c->nrow, nuc_rows * sizeof(lcs::NucRow))) != hipSuccess ||
         (e = hipMalloc(&c->nh_pk, nh_elems * 8)) != hipSuccess ||
         (e = hipMalloc(&c->nlist, nuc_rows * lcs::kNucList * 8)) != hipSuccess ||
@@ -601,8 +602,6 @@ int lcs_lmhead(lcs_ctx* c, const lcs_lmhead_batch* b, const lcs_lmhead_out* o, v
     a.rows = b->rows;
     a.vocab = b->vocab;
     a.hidden = b->hidden;
-    a.cols = lcs::lmhead_cols(b->vocab, c->cus);
-    a.nblocks = (b->vocab + a.cols - 1) / a.cols;
     a.rows_per_seq = b->rows_per_seq;
     a.ld_logits = o->ld_logits;
     a.draft = b->draft;
@@ -614,7 +613,7 @@ int lcs_lmhead(lcs_ctx* c, const lcs_lmhead_batch* b, const lcs_lmhead_out* o, v
     a.recs = c->lmrecs;
     a.stats = o->stats;
     DeviceGuard g(c->device);
-    const hipError_t e = lcs::launch_lmhead(a, static_cast<hipStream_t>(stream));
+    const hipError_t e = lcs::launch_lmhead(a, c->cus, static_cast<hipStream_t>(stream));
     if (e != hipSuccess) return hip_fail(c, e, "lm-head kernel launch");
     return LCS_OK;
 }

@@ -218,8 +218,7 @@ struct DraftArgs {
 };
 
 // lm-head product with the first statistics in its epilogue (lcs_lmhead.hip)
-constexpr uint32_t kLmRows = 64;    // rows per product launch (4 MFMA row tiles)
-constexpr uint32_t kLmColsMin = 256;  // vocabulary columns per workgroup (one record block): 256 or 320
+constexpr uint32_t kLmMaxBlocks = kMaxVocab / 256;  // column blocks (one record each) a row can have
 struct LmRec {                      // per (row, block of columns)
     float max;                      // the block's largest logit
     uint32_t idx;                   // its first column; bit 31: the block holds the row's draft token
@@ -230,9 +229,9 @@ constexpr uint32_t kLmDraftBit = 0x80000000u;
 struct LmArgs {
     const uint16_t* x;              // rows x hidden bf16
     const uint16_t* w;              // vocab x hidden bf16
-    uint32_t rows, vocab, hidden, m0, nblocks, rows_per_seq;
-    uint32_t cols;                  // columns per block (lmhead_cols)
-    uint32_t nchunks;               // 64-row chunks of one launch (see lmhead_kernel)
+    uint32_t rows, vocab, hidden, rows_per_seq;
+    uint32_t nblocks;               // column blocks and row tiles of the launch (launch_lmhead)
+    uint32_t nchunks;
     uint64_t ld_logits;             // elements between logits rows
     const int32_t* draft;
     float* logits;

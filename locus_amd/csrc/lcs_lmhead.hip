@@ -1,6 +1,6 @@
 // The lm-head product with the sampler's first statistics in its epilogue,
 // for MI355X (gfx950): logits = X W^T in bf16 on the matrix cores (f32
-// accumulation), and per (row, block of 256 vocabulary columns) the block's
+// accumulation), and per (row, block of vocabulary columns) the block's
 // argmax (first index), its sum of exponentials against the block max, and
 // the logit of the row's draft token when the block holds it. A per-sequence
 // finalize then gives each row's argmax and log-normaliser, the draft's
@@ -14,20 +14,17 @@
 // logprobs_from with chosen = draft (sampling.cpp:150-170) per row and the
 // acceptance rule of engine.cpp:357-383 per sequence.
 //
-// Tiling: a workgroup of four waves computes 64 rows x 256 columns; each wave
-// holds 4 x 4 tiles of 16 x 16 (v_mfma_f32_16x16x32_bf16: lane l carries
-// 8 consecutive k of row l % 16 of A, the same k of column l % 16 of B, and
-// returns rows 4 (l / 16) + i of column l % 16 of C). The weight (W, the
-// K-contiguous vocab-major matrix) comes straight from HBM into registers,
-// 16 bytes per lane per fragment, 128 contiguous bytes of each of a wave's
-// 64 rows per k-step, three k-steps in flight; x (shared by the four waves)
-// is staged through LDS. Every weight byte is read once per launch of up to
-// 64 rows: the weight stream is the bound for decode batches.
+// Up to 64 rows (decode) the weight stream from HBM is the bound; from 256
+// rows up (verify) the matrix cores are.
 //
-// Measured (64 x 128256 x 4096, MI355X): the fused launch takes about as long
-// as the library GEMM alone writing bf16 logits, and less than that GEMM
-// followed by the verify kernels. Shapes whose block count lands just above
-// the 512 resident workgroups (two per CU) pay a tail round.
+// Measured (us a call; the library bf16 GEMM alone 976 at 1024 rows; "before":
+// this kernel's predecessor, 64 rows x 256 columns with the weight fragments
+// loaded straight into registers and the shared x behind a barrier per step):
+//   rows x columns x hidden       before   now
+//   64   x 128256 x 4096 (logits)   217    203
+//   8    x 32000  x 4096            124     51
+//   128  x 128256 x 4096            448    220
+//   1024 x 128256 x 4096           2629    975
 #include <hip/hip_runtime.h>
 #include <math.h>
 #include <stdint.h>
@@ -39,270 +36,323 @@ namespace lcs {
 
 namespace {
 typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
-typedef float f32x4 __attribute__((ext_vector_type(4)));
+typedef float f32x16 __attribute__((ext_vector_type(16)));
 constexpr int kLmThreads = 256;
 constexpr float kL2E = 1.4426950408889634f;
-constexpr int kKC = 2;      // 32-wide k chunks per step: 128 bytes of each weight row
+constexpr int kTK = 32;                       // k per LDS stage
+constexpr uint32_t kTRowB = kTK * 2;          // bytes of a row in a stage
+constexpr uint32_t kBigHidden = 1u << 22;     // above: 64-bit row offsets
 
-__device__ __forceinline__ bf16x8 ld_frag(const uint16_t* p) {
-    return __builtin_bit_cast(bf16x8, *reinterpret_cast<const uint4*>(p));
+// Waits until at most N vector memory operations are outstanding (and every
+// LDS operation is done); the compiler moves no memory access across it.
+template <int N>
+__device__ __forceinline__ void wait_vm() {
+    asm volatile("s_waitcnt vmcnt(%0)" ::"n"(N) : "memory");
+}
+template <int N>
+__device__ __forceinline__ void wait_vm_lgkm() {
+    asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)" ::"n"(N) : "memory");
 }
 
-// Lanes 16q .. 16q+15 (a DPP row) end holding the row's minimum of the
-// 64-bit keys (quad_perm [1,0,3,2], [2,3,0,1], row_half_mirror, row_mirror).
-__device__ __forceinline__ uint64_t row16_min_u64(uint64_t v) {
-    v = u64_min(v, dpp_u64<0xB1>(~0ull, v));
-    v = u64_min(v, dpp_u64<0x4E>(~0ull, v));
-    v = u64_min(v, dpp_u64<0x141>(~0ull, v));
-    v = u64_min(v, dpp_u64<0x140>(~0ull, v));
-    return v;
+// 16 bytes per lane from a buffer (offsets vo per lane + so) to LDS at
+// dst + 16 lane (dst is wave-uniform).
+__device__ __forceinline__ void dma16(__amdgpu_buffer_rsrc_t rs, unsigned char* dst, uint32_t vo, uint32_t so) {
+    __builtin_amdgcn_raw_ptr_buffer_load_lds(rs, (__attribute__((address_space(3))) void*)dst, 16, (int)vo, (int)so, 0, 0);
 }
-__device__ __forceinline__ float row16_sum(float v) {
-    v += __int_as_float(dpp_i<0xB1>(0, __float_as_int(v)));
-    v += __int_as_float(dpp_i<0x4E>(0, __float_as_int(v)));
-    v += __int_as_float(dpp_i<0x141>(0, __float_as_int(v)));
-    v += __int_as_float(dpp_i<0x140>(0, __float_as_int(v)));
-    return v;
+// The same from a per-lane address.
+__device__ __forceinline__ void dma16_at(const void* src, unsigned char* dst) {
+    __builtin_amdgcn_global_load_lds((const __attribute__((address_space(1))) void*)src,
+                                     (__attribute__((address_space(3))) void*)dst, 16, 0, 0);
 }
+// A workgroup barrier that waits for no memory operation.
+__device__ __forceinline__ void block_sync() {
+    __builtin_amdgcn_sched_barrier(0);
+    __builtin_amdgcn_s_barrier();
+    asm volatile("" ::: "memory");
+    __builtin_amdgcn_sched_barrier(0);
+}
+
 }  // namespace
 
-// A workgroup computes one block of columns for one chunk of <= kLmRows
-// rows. With one chunk (a.nchunks 1) workgroup w takes block w of chunk
-// a.m0. With several, one launch covers every chunk, and the workgroups of a
-// block are placed on one XCD in consecutive dispatch slots (workgroups are
-// dealt to the 8 XCDs in turn): they run together, so the block's weight rows
-// come from HBM once and from that XCD's L2 for the other chunks. WC: 16-column
-// MFMA tiles per wave (the workgroup's block is 64 WC columns); kDepth:
-// weight k-steps in flight ahead of the product.
-template <int WC, int kDepth>
-__global__ __launch_bounds__(kLmThreads, 2) void lmhead_kernel(LmArgs a) {
-    __shared__ uint64_t pkey[kLmThreads / kWave][kLmRows];   // per wave: row's best (rank key)
-    __shared__ float psum[kLmThreads / kWave][kLmRows];
-    __shared__ float pdraft[kLmRows];
-    __shared__ uint32_t pfound[kLmRows];
+// A workgroup computes 64 VT columns of BR rows, transposed (columns on the
+// MFMA's row side, so that a lane holds many columns of one row and the
+// epilogue reduces in registers): four waves of 32 VT columns x BR / 2 rows in
+// v_mfma_f32_32x32x16_bf16 tiles (lane l carries 8 consecutive k of row l % 32
+// of either operand, k chunk l / 32, and returns rows 8 (e / 4) + 4 (l / 32) +
+// e % 4 of column l % 32).
+//
+// Both operands go straight from memory into a ring of ST LDS stages of 32 k
+// with 16-byte DMA loads, so that no register holds data in flight and ST - 1
+// stages are (a stage is 64 bytes of each row). A row's four 16-byte chunks are
+// permuted by bits 2-3 of the row: a fragment read's 16 lanes of a phase then
+// cover the 64 banks once (0 conflict cycles of 67 M; permuted by bits 1-2,
+// half of 133 M). One barrier per stage, in the middle of its products: each
+// wave has then read the stage and its loads of the next one have landed.
+//
+// The workgroups of a column block are placed on one XCD in consecutive
+// dispatch slots (workgroups are dealt to the 8 XCDs in turn): they run
+// together, so the block's weight rows come from HBM once and from that XCD's
+// L2 for the other row tiles. With one row tile each workgroup starts at its
+// own k-step and wraps round, so that those in flight do not all read the same
+// offset of their rows (72 rows x 128256 x 4096: 245 -> 225 us); with more the
+// row tiles share x through the L2 by running in step (1024 rows: 1013 against
+// 1057 us with a start of its own).
+template <int VT, int BR, int ST, bool BIG = false>
+__global__ __launch_bounds__(kLmThreads, VT * BR == 1024 ? 1 : 2) void lmhead_tile(LmArgs a) {
+    constexpr uint32_t kTV = 64u * VT;        // columns per workgroup
+    constexpr uint32_t kStage = (kTV + BR) * kTRowB;
+    constexpr int RT = BR / 64;               // 32-row tiles per wave
+    constexpr int LA = kTV / 64, LB = BR / 64;   // DMA loads per wave and stage
+    constexpr int LPS = LA + LB;
+    __shared__ __attribute__((aligned(128))) unsigned char lds[ST * kStage];
     const uint32_t tid = tid_x();
-    const int lane = lane_id(), wv = (int)(tid / kWave);
-    uint32_t nb = wg_x(), m0 = a.m0;
-    if (a.nchunks > 1u) {
-        const uint32_t slot = nb >> 3;
-        m0 = (slot % a.nchunks) * kLmRows;
-        nb = 8u * (slot / a.nchunks) + (nb & 7u);
-        if (nb >= a.nblocks) return;   // (the grid is a multiple of 8 blocks)
-    }
+    const int lane = lane_id(), wv = __builtin_amdgcn_readfirstlane((int)(tid / kWave));
+    uint32_t nb = wg_x();
+    const uint32_t slot = nb >> 3;
+    const uint32_t r0 = (slot % a.nchunks) * BR;
+    nb = 8u * (slot / a.nchunks) + (nb & 7u);
+    if (nb >= a.nblocks) return;   // (the grid is a multiple of 8 blocks)
     const uint32_t K = a.hidden, V = a.vocab;
-    const uint32_t mrows = min((uint32_t)kLmRows, a.rows - m0);
-    constexpr uint32_t kCols = 4u * 16u * WC;
-    const uint32_t nw = nb * kCols + (uint32_t)wv * (16u * WC);   // this wave's first column
-    const uint32_t lr = (uint32_t)lane & 15u, kq = (uint32_t)lane >> 4;
-    // fragment rows: A rows past the chunk and B columns past the vocabulary
-    // read row 0 / column 0 (in bounds) and are masked in the epilogue
-    const uint16_t* xr[4];
-    const uint16_t* wr[WC];
+    const uint32_t n0 = nb * kTV;
+    const uint32_t vrows = min((uint32_t)BR, a.rows - r0), vcols = min(kTV, V - n0);
+    const uint32_t wm = (uint32_t)wv & 1u, wn = (uint32_t)wv >> 1;   // the wave's columns and rows
+    const uint16_t* wbase = a.w + (uint64_t)n0 * K;
+    const uint16_t* xbase = a.x + (uint64_t)r0 * K;
+    const __amdgpu_buffer_rsrc_t wrs =
+        __builtin_amdgcn_make_buffer_rsrc(const_cast<uint16_t*>(wbase), 0, (int)(vcols * K * 2u), 0x00020000);
+    const __amdgpu_buffer_rsrc_t xrs =
+        __builtin_amdgcn_make_buffer_rsrc(const_cast<uint16_t*>(xbase), 0, (int)(vrows * K * 2u), 0x00020000);
+    // DMA load i of a wave covers rows 64 i + 16 wv + lane / 4, a 16-byte
+    // chunk per lane; rows past the tile read row 0 (masked in the epilogue)
+    const uint32_t rr = 16u * (uint32_t)wv + ((uint32_t)lane >> 2);
+    const uint32_t ch = (((uint32_t)lane & 3u) ^ ((rr >> 2) & 3u)) * 16u;
+    uint32_t wo[LA], xo[LB];
 #pragma unroll
-    for (int t = 0; t < 4; ++t) {
-        const uint32_t r = (uint32_t)t * 16u + lr;
-        xr[t] = a.x + (uint64_t)(m0 + (r < mrows ? r : 0u)) * K + kq * 8u;
+    for (int i = 0; i < LA; ++i) wo[i] = (64u * i + rr < vcols ? 64u * i + rr : 0u) * K * 2u + ch;
+#pragma unroll
+    for (int i = 0; i < LB; ++i) xo[i] = (64u * i + rr < vrows ? 64u * i + rr : 0u) * K * 2u + ch;
+    const uint32_t nsteps = K / kTK;
+    const uint32_t rot = a.nchunks == 1u ? nb % nsteps : 0u;
+    // (the byte offset of stage t in a row; stages past the end re-read the last)
+    auto koff = [&](uint32_t t) -> uint32_t {
+        uint32_t q = (t < nsteps ? t : nsteps - 1u) + rot;
+        return (q >= nsteps ? q - nsteps : q) * kTRowB;
+    };
+    auto issue1 = [&](int i, uint32_t ko, uint32_t sl) {   // DMA load i of a stage
+        unsigned char* b = lds + sl * kStage + (uint32_t)wv * 1024u + i * 4096;
+        if (BIG) {   // (the row offsets need 64 bits)
+            const uint32_t r = 64u * (uint32_t)(i < LA ? i : i - LA) + rr;
+            const uint16_t* p = i < LA ? wbase + (uint64_t)(r < vcols ? r : 0u) * K : xbase + (uint64_t)(r < vrows ? r : 0u) * K;
+            dma16_at(reinterpret_cast<const unsigned char*>(p) + ko + ch, b);
+        } else if (i < LA) {
+            dma16(wrs, b, wo[i < LA ? i : 0], ko);
+        } else {
+            dma16(xrs, b, xo[i >= LA ? i - LA : 0], ko);
+        }
+    };
+    auto issue = [&](uint32_t t, uint32_t sl) {
+#pragma unroll
+        for (int i = 0; i < LPS; ++i) issue1(i, koff(t), sl);
+    };
+    f32x16 acc[VT][RT];
+#pragma unroll
+    for (int i = 0; i < VT; ++i)
+#pragma unroll
+        for (int j = 0; j < RT; ++j)
+#pragma unroll
+            for (int e = 0; e < 16; ++e) acc[i][j][e] = 0.0f;
+    // fragment s (16 k) of row r: chunk 2 s + lane / 32
+    const uint32_t lr = (uint32_t)lane & 31u, lh = (uint32_t)lane >> 5;
+    uint32_t fo[2];
+#pragma unroll
+    for (uint32_t s = 0; s < 2; ++s) fo[s] = lr * kTRowB + (((2u * s + lh) ^ ((lr >> 2) & 3u)) * 16u);
+    struct Frag { bf16x8 w[VT], x[RT]; };
+    // read i of a fragment set: x first (every product needs all of it), then w
+    constexpr int NR = VT + RT, NP = VT * RT;
+    auto read1 = [&](Frag& f, int i, uint32_t sl, int s) {
+        const unsigned char* pw = lds + sl * kStage + wm * (kTV / 2 * kTRowB) + fo[s];
+        const unsigned char* px = lds + sl * kStage + kTV * kTRowB + wn * (BR / 2 * kTRowB) + fo[s];
+        if (i < RT) f.x[i < RT ? i : 0] = *reinterpret_cast<const bf16x8*>(px + i * 32 * kTRowB);
+        else f.w[i >= RT ? i - RT : 0] = *reinterpret_cast<const bf16x8*>(pw + (i - RT) * 32 * kTRowB);
+    };
+    auto mul1 = [&](const Frag& f, int k) {   // product k of NP
+        const int i = k / RT, j = k % RT;
+        acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(f.w[i], f.x[j], acc[i][j], 0, 0, 0);
+    };
+    Frag f0, f1;
+#pragma unroll
+    for (int t = 0; t < ST; ++t) issue((uint32_t)t, (uint32_t)t);
+    wait_vm<(ST - 1) * LPS>();
+    block_sync();
+#pragma unroll
+    for (int i = 0; i < NR; ++i) read1(f0, i, 0u, 0);
+    uint32_t sl = 0u;
+    // Every LDS read and DMA load is issued behind a product: a wave issues
+    // in order, and eight DMA loads in a row hold it for longer than the
+    // products queued ahead of them last (1024 rows: 1022 -> 980 us).
+    for (uint32_t t = 0; t < nsteps; ++t) {
+        const uint32_t ns = sl + 1u == (uint32_t)ST ? 0u : sl + 1u;
+#pragma unroll
+        for (int k = 0; k < NP; ++k) {
+            mul1(f0, k);
+#pragma unroll
+            for (int i = k * NR / NP; i < (k + 1) * NR / NP; ++i) read1(f1, i, sl, 1);
+            __builtin_amdgcn_sched_barrier(0);
+        }
+        // stage t is read, stage t + 1 has landed, in every wave
+        wait_vm_lgkm<(ST - 2) * LPS>();
+        block_sync();
+        const uint32_t ko = koff(t + ST);
+#pragma unroll
+        for (int k = 0; k < NP; ++k) {
+            mul1(f1, k);
+#pragma unroll
+            for (int i = k * (NR + LPS) / NP; i < (k + 1) * (NR + LPS) / NP; ++i) {
+                if (i < NR) read1(f0, i, ns, 0);
+                else issue1(i - NR, ko, sl);
+            }
+            __builtin_amdgcn_sched_barrier(0);
+        }
+        sl = ns;
     }
-#pragma unroll
-    for (int t = 0; t < WC; ++t) {
-        const uint32_t c = nw + (uint32_t)t * 16u + lr;
-        wr[t] = a.w + (uint64_t)(c < V ? c : 0u) * K + kq * 8u;
-    }
-    f32x4 acc[4][WC];
-#pragma unroll
-    for (int i = 0; i < 4; ++i)
-#pragma unroll
-        for (int j = 0; j < WC; ++j) acc[i][j] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
-    // k-steps of 32 kKC wide. The weight fragments (the HBM stream, each
-    // wave its own columns) are software-pipelined kDepth steps deep in
-    // registers: those of step s + kDepth are requested while step s
-    // multiplies (a ring of kDepth + 1 buffers). The x fragments are common
-    // to the four waves: wave w fetches row tile w of step s + 1 during step
-    // s and stores it in an LDS double buffer (fragment-major, lane l's
-    // 16 bytes at l * 16, so reads and writes are conflict-free), from which
-    // every wave reads its A operands after the step's barrier. Every load is
-    // unconditional (steps past the end re-read the last one). Each
-    // workgroup starts at its own k-step (rot) and wraps round, so that the
-    // workgroups in flight do not all read the same offset of their rows.
-    const uint32_t nsteps = K / (32u * kKC);
-    const uint32_t rot = nb % nsteps;
-    auto koff = [&](uint32_t st) -> uint32_t {
-        uint32_t q = (st < nsteps ? st : nsteps - 1u) + rot;
-        q = q >= nsteps ? q - nsteps : q;
-        return q * 32u * kKC;
-    };
-    constexpr int NB = kDepth + 1;
-    constexpr uint32_t kXFrag = kWave * 16u;            // bytes per fragment
-    constexpr uint32_t kXBuf = 4u * kKC * kXFrag;       // bytes per step
-    __shared__ __attribute__((aligned(16))) unsigned char xs[2 * kXBuf];
-    const uint16_t* xw = xr[wv];                        // this wave's x row tile
-    bf16x8 bw[NB][kKC][WC], xv[kKC], af[kKC][4];
-    auto load_w = [&](int buf, uint32_t st) {
-        const uint32_t ko = koff(st);
-#pragma unroll
-        for (int c = 0; c < kKC; ++c)
-#pragma unroll
-            for (int t = 0; t < WC; ++t) bw[buf][c][t] = ld_frag(wr[t] + ko + 32u * c);
-    };
-    auto load_x = [&](uint32_t st) {
-        const uint32_t ko = koff(st);
-#pragma unroll
-        for (int c = 0; c < kKC; ++c) xv[c] = ld_frag(xw + ko + 32u * c);
-    };
-    auto put_x = [&](uint32_t st) {
-        unsigned char* b = xs + (st & 1u) * kXBuf + (uint32_t)lane * 16u;
-#pragma unroll
-        for (int c = 0; c < kKC; ++c)
-            *reinterpret_cast<bf16x8*>(b + ((uint32_t)wv * kKC + c) * kXFrag) = xv[c];
-    };
-    auto get_x = [&](uint32_t st) {
-        const unsigned char* b = xs + (st & 1u) * kXBuf + (uint32_t)lane * 16u;
-#pragma unroll
-        for (int t = 0; t < 4; ++t)
-#pragma unroll
-            for (int c = 0; c < kKC; ++c)
-                af[c][t] = *reinterpret_cast<const bf16x8*>(b + ((uint32_t)t * kKC + c) * kXFrag);
-    };
-    auto step = [&](int u, uint32_t st) {
-        load_x(st + 1u);
-        load_w((u + kDepth) % NB, st + kDepth);
-        get_x(st);
-#pragma unroll
-        for (int c = 0; c < kKC; ++c)
-#pragma unroll
-            for (int i = 0; i < 4; ++i)
-#pragma unroll
-                for (int j = 0; j < WC; ++j)
-                    acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(af[c][i], bw[u][c][j], acc[i][j], 0, 0, 0);
-        put_x(st + 1u);
-        __syncthreads();
-    };
-    load_x(0u);
-#pragma unroll
-    for (int u = 0; u < kDepth; ++u) load_w(u, (uint32_t)u);
-    put_x(0u);
-    __syncthreads();
-    const uint32_t nfull = nsteps / NB * NB;
-    for (uint32_t s0 = 0; s0 < nfull; s0 += NB) {
-#pragma unroll
-        for (int u = 0; u < NB; ++u) step(u, s0 + (uint32_t)u);
-    }
-    // the remaining steps (fewer than NB): their weights were requested by
-    // the loop's last round (or the prologue) into buffers 0, 1, ...
-#pragma unroll
-    for (int u = 0; u < NB - 1; ++u) {
-        if (nfull + (uint32_t)u < nsteps) step(u, nfull + (uint32_t)u);
-    }
+    wait_vm_lgkm<0>();
+    __syncthreads();   // (the last loads have landed: the ring is free)
 
-    // ---- epilogue: acc[i][j][e] is row 16 i + 4 kq + e, column nw + 16 j + lr
-    if (tid < kLmRows) { pdraft[tid] = 0.0f; pfound[tid] = 0u; }
-    if (a.logits) {
+    // ---- epilogue: acc[i][j][e] is column n0 + kTV / 2 wm + 32 i + 8 (e / 4) +
+    // 4 lh + e % 4 of row r0 + BR / 2 wn + 32 j + lr ----
+    struct Part { float max, sum, draft; uint32_t idx; };
+    Part* part = reinterpret_cast<Part*>(lds);   // [2][BR]: by the wave's columns
+    const bool full = vcols == kTV;
+    const bool vec = a.logits && (a.ld_logits & 3u) == 0u && (reinterpret_cast<uintptr_t>(a.logits) & 15u) == 0u;
 #pragma unroll
-        for (int i = 0; i < 4; ++i)
+    for (int j = 0; j < RT; ++j) {
+        const uint32_t rl = wn * (BR / 2) + 32u * j + lr;   // the lane's row in the tile
+        const bool rin = rl < vrows;
+        const uint32_t cb = kTV / 2 * wm + 4u * lh;            // columns cb + 32 i + 8 (e / 4) + e % 4
+        if (a.logits && rin) {
+            float* out = a.logits + (uint64_t)(r0 + rl) * a.ld_logits + n0;
 #pragma unroll
-            for (int e = 0; e < 4; ++e) {
-                const uint32_t r = (uint32_t)i * 16u + kq * 4u + (uint32_t)e;
-                if (r < mrows) {
-                    float* out = a.logits + (uint64_t)(m0 + r) * a.ld_logits;
+            for (int i = 0; i < VT; ++i)
 #pragma unroll
-                    for (int j = 0; j < WC; ++j) {
-                        const uint32_t c = nw + (uint32_t)j * 16u + lr;
-                        if (c < V) out[c] = acc[i][j][e];
+                for (int q = 0; q < 4; ++q) {
+                    const uint32_t c = cb + 32u * i + 8u * q;
+                    if (vec && c + 4u <= vcols) {
+                        *reinterpret_cast<float4*>(out + c) =
+                            make_float4(acc[i][j][4 * q], acc[i][j][4 * q + 1], acc[i][j][4 * q + 2], acc[i][j][4 * q + 3]);
+                    } else {
+#pragma unroll
+                        for (int e = 0; e < 4; ++e)
+                            if (c + e < vcols) out[c + e] = acc[i][j][4 * q + e];
                     }
                 }
+        }
+        const float NEG = -__builtin_huge_valf();
+        if (!full) {
+#pragma unroll
+            for (int i = 0; i < VT; ++i)
+#pragma unroll
+                for (int e = 0; e < 16; ++e)
+                    if (cb + 32u * i + 8u * (e / 4) + e % 4 >= vcols) acc[i][j][e] = NEG;
+        }
+        // the lane's max, its first column, the draft's logit
+        float m = acc[0][j][0];
+#pragma unroll
+        for (int i = 0; i < VT; ++i)
+#pragma unroll
+            for (int e = 0; e < 16; ++e) m = fmaxf(m, acc[i][j][e]);
+        const int32_t dr = a.draft && rin ? a.draft[r0 + rl] : -1;
+        const uint32_t dc = (uint32_t)dr < V ? (uint32_t)dr - n0 - cb : 0xffffffffu;   // the draft's column, from cb
+        uint32_t ci = kTV;
+        float dl = 0.0f;
+#pragma unroll
+        for (int i = VT - 1; i >= 0; --i)
+#pragma unroll
+            for (int e = 15; e >= 0; --e) {
+                const uint32_t c = 32u * i + 8u * (e / 4) + e % 4;
+                ci = acc[i][j][e] == m ? c : ci;
             }
-    }
-    __syncthreads();   // (pdraft initialised)
-    // per row: this wave's best (value, first column) over its 64 columns, as
-    // a rank key (value descending, column ascending)
+        uint32_t found = 0u;
+        if (ballot(dc < kTV / 2 && (dc & 4u) == 0u) != 0u) {
 #pragma unroll
-    for (int i = 0; i < 4; ++i)
+            for (int i = 0; i < VT; ++i)
 #pragma unroll
-        for (int e = 0; e < 4; ++e) {
-            const uint32_t r = (uint32_t)i * 16u + kq * 4u + (uint32_t)e;
-            uint64_t best = ~0ull;
-            const int32_t dr = (a.draft && r < mrows) ? a.draft[m0 + r] : -1;
-#pragma unroll
-            for (int j = 0; j < WC; ++j) {
-                const uint32_t c = nw + (uint32_t)j * 16u + lr;
-                if (c < V) {
-                    const uint64_t k = rank_key(acc[i][j][e], c);
-                    best = k < best ? k : best;
-                    if ((int32_t)c == dr) { pdraft[r] = acc[i][j][e]; pfound[r] = kLmDraftBit; }
+                for (int e = 0; e < 16; ++e) {
+                    const uint32_t c = 32u * i + 8u * (e / 4) + e % 4;
+                    if (dc == c) { dl = acc[i][j][e]; found = kLmDraftBit; }
                 }
+        }
+        ci += cb;
+        // (a lane whose columns all lie past the vocabulary: max -inf, no term)
+        float s = 0.0f;
+#pragma unroll
+        for (int i = 0; i < VT; ++i)
+#pragma unroll
+            for (int e = 0; e < 16; e += 4) {
+                float t[4];
+#pragma unroll
+                for (int k = 0; k < 4; ++k) t[k] = __builtin_amdgcn_exp2f((acc[i][j][e + k] - m) * kL2E);
+                s += (t[0] + t[1]) + (t[2] + t[3]);
             }
-            best = row16_min_u64(best);
-            if (lr == 0u) pkey[wv][r] = best;
-        }
+        s = m == NEG ? 0.0f : s;
+        // lanes l and l + 32 share a row
+        const float m2 = __shfl_xor(m, 32), s2 = __shfl_xor(s, 32), d2 = __shfl_xor(dl, 32);
+        const uint32_t c2 = (uint32_t)__shfl_xor((int)ci, 32), f2 = (uint32_t)__shfl_xor((int)found, 32);
+        const float M = fmaxf(m, m2);
+        s = (m == NEG ? 0.0f : s * __builtin_amdgcn_exp2f((m - M) * kL2E)) +
+            (m2 == NEG ? 0.0f : s2 * __builtin_amdgcn_exp2f((m2 - M) * kL2E));
+        ci = m > m2 ? ci : m2 > m ? c2 : min(ci, c2);
+        if (lh == 0u) part[wm * BR + rl] = Part{M, s, found ? dl : d2, ci | found | f2};
+    }
     __syncthreads();
-    // the block's max per row (all four waves' keys), then sums of exp(v - max)
-    float bmax[4][4];
-#pragma unroll
-    for (int i = 0; i < 4; ++i)
-#pragma unroll
-        for (int e = 0; e < 4; ++e) {
-            const uint32_t r = (uint32_t)i * 16u + kq * 4u + (uint32_t)e;
-            const uint64_t k = u64_min(u64_min(pkey[0][r], pkey[1][r]), u64_min(pkey[2][r], pkey[3][r]));
-            bmax[i][e] = rank_val(k);
-        }
-#pragma unroll
-    for (int i = 0; i < 4; ++i)
-#pragma unroll
-        for (int e = 0; e < 4; ++e) {
-            const uint32_t r = (uint32_t)i * 16u + kq * 4u + (uint32_t)e;
-            // (v - max) first: it is exact or nearly so, where a fused
-            // v * log2(e) - max * log2(e) would carry the rounding of the
-            // large product max * log2(e) into every term
-            const float bm = bmax[i][e];
-            float s = 0.0f;
-#pragma unroll
-            for (int j = 0; j < WC; ++j) {
-                const uint32_t c = nw + (uint32_t)j * 16u + lr;
-                if (c < V) s += __builtin_amdgcn_exp2f((acc[i][j][e] - bm) * kL2E);
-            }
-            s = row16_sum(s);
-            if (lr == 0u) psum[wv][r] = s;
-        }
-    __syncthreads();
-    // one record per row of the chunk
-    if (tid < mrows) {
-        const uint32_t r = tid;
-        const uint64_t k = u64_min(u64_min(pkey[0][r], pkey[1][r]), u64_min(pkey[2][r], pkey[3][r]));
+    if (tid < vrows) {
+        const Part p = part[tid], q = part[BR + tid];
+        const float NEG = -__builtin_huge_valf();
+        const float M = fmaxf(p.max, q.max);
         LmRec rec;
-        rec.max = rank_val(k);
-        rec.idx = rank_idx(k) | pfound[r];
-        rec.sum = (psum[0][r] + psum[1][r]) + (psum[2][r] + psum[3][r]);
-        rec.draft = pdraft[r];
-        a.recs[(uint64_t)(m0 + r) * a.nblocks + nb] = rec;
+        rec.max = M;
+        // (equal maxima: the lower columns are p's)
+        rec.idx = (n0 + ((p.max >= q.max ? p.idx : q.idx) & ~kLmDraftBit)) | ((p.idx | q.idx) & kLmDraftBit);
+        rec.sum = p.sum * __builtin_amdgcn_exp2f((p.max - M) * kL2E) +
+                  (q.max == NEG ? 0.0f : q.sum * __builtin_amdgcn_exp2f((q.max - M) * kL2E));
+        rec.draft = (p.idx & kLmDraftBit) ? p.draft : q.draft;
+        a.recs[(uint64_t)(r0 + tid) * a.nblocks + nb] = rec;
     }
 }
 
 // One workgroup per sequence (rows_per_seq rows; a row is its own sequence
-// when rows_per_seq is 0): wave w merges rows w, w + 4, ... from their
-// blocks' records (the kernel boundary orders them after the product).
-__global__ __launch_bounds__(kLmThreads) void lmhead_fin(LmArgs a) {
+// when rows_per_seq is 0): wave w of NW merges rows w, w + NW, ... from their
+// blocks' records (the kernel boundary orders them after the product). A row's
+// records (at most 64 PER) are requested together and stay in registers: one
+// memory round trip a row (1024 rows of 501 records: 13.2 -> 5.6 us).
+template <int NW, uint32_t PER>
+__global__ __launch_bounds__(NW * kWave) void lmhead_fin(LmArgs a) {
     __shared__ int32_t am[64];
     const uint32_t tid = tid_x();
     const int lane = lane_id(), wv = (int)(tid / kWave);
     const uint32_t R = a.rows_per_seq ? a.rows_per_seq : 1u;
     const uint32_t seq = wg_x();
-    for (uint32_t j = (uint32_t)wv; j < R; j += kLmThreads / kWave) {
+    for (uint32_t j = (uint32_t)wv; j < R; j += NW) {
         const uint32_t row = seq * R + j;
         const LmRec* rr = a.recs + (uint64_t)row * a.nblocks;
-        uint64_t best = ~0ull;
-        for (uint32_t b = (uint32_t)lane; b < a.nblocks; b += kWave) {
-            const uint64_t k = rank_key(rr[b].max, rr[b].idx & ~kLmDraftBit);
-            best = k < best ? k : best;
+        LmRec rc[PER];
+#pragma unroll
+        for (uint32_t i = 0; i < PER; ++i) {   // (past the end: block 0 again)
+            const uint32_t b = i * kWave + (uint32_t)lane;
+            rc[i] = rr[b < a.nblocks ? b : 0u];
         }
+        uint64_t best = ~0ull;
+#pragma unroll
+        for (uint32_t i = 0; i < PER; ++i) best = u64_min(best, rank_key(rc[i].max, rc[i].idx & ~kLmDraftBit));
         best = wave_min_u64(best);
         const float M = rank_val(best);
         double z = 0.0;
         float dl = 0.0f;
         bool has = false;
-        for (uint32_t b = (uint32_t)lane; b < a.nblocks; b += kWave) {
-            const LmRec rc = rr[b];
-            z += (double)rc.sum * (double)__builtin_amdgcn_exp2f((rc.max - M) * kL2E);
-            if (rc.idx & kLmDraftBit) { dl = rc.draft; has = true; }
+#pragma unroll
+        for (uint32_t i = 0; i < PER; ++i) {
+            const bool in = i * kWave + (uint32_t)lane < a.nblocks;
+            z += in ? (double)rc[i].sum * (double)__builtin_amdgcn_exp2f((rc[i].max - M) * kL2E) : 0.0;
+            if (in && (rc[i].idx & kLmDraftBit)) { dl = rc[i].draft; has = true; }
         }
         z = wave_sum(z);
         const uint64_t own = ballot(has);
@@ -325,32 +375,82 @@ __global__ __launch_bounds__(kLmThreads) void lmhead_fin(LmArgs a) {
     }
 }
 
-// The block shape per launch: 256 columns three k-steps deep, or 320
-// columns two k-steps deep (the register budget of two workgroups per CU)
-// when that fits the blocks in one round of resident workgroups and 256
-// does not (a vocabulary just above 512 blocks of 256 would pay a second,
-// mostly idle round).
-uint32_t lmhead_cols(uint32_t vocab, uint32_t cus) {
-    const uint32_t slots = 2u * (cus ? cus : 256u);
-    const uint32_t n4 = (vocab + 255u) / 256u, n5 = (vocab + 319u) / 320u;
-    const uint32_t r4 = (n4 + slots - 1u) / slots, r5 = (n5 + slots - 1u) / slots;
-    return r5 < r4 ? 320u : 256u;
+// Column blocks of 64 vt columns that a context's record buffer has to hold for
+// a vocabulary (see lmhead_shape's limits).
+uint32_t lmhead_max_blocks(uint32_t vocab, uint32_t cus) {
+    auto n = [&](uint32_t c) { return (vocab + c - 1u) / c; };
+    auto least = [](uint32_t a, uint32_t b) { return a < b ? a : b; };
+    const uint32_t n1 = least(n(64u), cus * 2u), n2 = least(n(128u), cus * 4u);
+    const uint32_t m = least(n1 > n2 ? n1 : n2, kLmMaxBlocks);
+    return m > n(256u) ? m : n(256u);
 }
 
-hipError_t launch_lmhead(const LmArgs& a0, hipStream_t st) {
-    LmArgs a = a0;
-    const bool wide = a0.cols == 320u;
-    a.m0 = 0;
-    a.nchunks = (a0.rows + kLmRows - 1) / kLmRows;
-    const uint32_t grid = a.nchunks > 1u ? 8u * ((a.nblocks + 7u) / 8u) * a.nchunks : a.nblocks;
-    if (wide) hipLaunchKernelGGL((lmhead_kernel<5, 2>), dim3(grid), dim3(kLmThreads), 0, st, a);
-    else hipLaunchKernelGGL((lmhead_kernel<4, 3>), dim3(grid), dim3(kLmThreads), 0, st, a);
-    {
-        const hipError_t e = hipGetLastError();
-        if (e != hipSuccess) return e;
+// The tile of a launch. Rows: 64-row tiles up to 64 rows; above, a 128-row tile
+// where that leaves out a 256-row tile more than half empty (128 rows: 225
+// against 288 us, 384 rows: 479 against 505; 256 rows: 357 against 308).
+// Columns: a CU runs its workgroups' columns one after the other, whether two
+// are resident or one, so the time goes by ceil(workgroups / CUs) x columns;
+// narrow tiles read x more often for the same columns (64 x 128256 x 4096,
+// 2 x 256, 4 x 128 and 8 x 64 columns a CU: 209, 227, 276 us), hence the
+// weights. 64 rows x 4096, us by 320 / 256 / 128 / 64 columns (the rule's
+// first): 20000: 51 (128), 62, 72; 40000: 89 (256), 99, 102; 80000: 131
+// (320), 156, 162, 169; 128256: 209 (256), 226, 271; 151936 x 3584: 224 (320),
+// 249, 251, 325.
+struct LmShape { uint32_t vt, br; };
+static LmShape lmhead_shape(uint32_t rows, uint32_t vocab, uint32_t hidden, uint32_t cus) {
+    if (hidden > kBigHidden) return {4u, 64u};
+    const uint32_t br = rows <= 64u ? 64u : rows <= 128u || (rows > 256u && rows <= 384u) ? 128u : 256u;
+    const uint32_t chunks = (rows + br - 1u) / br;
+    struct { uint32_t vt, br, weight; } const shapes[] = {   // (widest first; weight in 1/64)
+        {5, 64, 64}, {4, 64, 64}, {2, 64, 69}, {1, 64, 85}, {4, 128, 64}, {2, 128, 77}, {4, 256, 64}, {2, 256, 77}};
+    LmShape best{4u, br};
+    uint64_t least = ~0ull;
+    for (const auto& s : shapes) {
+        if (s.br != br) continue;
+        const uint64_t n = ((uint64_t)vocab + 64u * s.vt - 1u) / (64u * s.vt);
+        if ((s.vt == 1u && n > 2u * cus) || (s.vt == 2u && n > 4u * cus) || n > kLmMaxBlocks) continue;   // (lmhead_max_blocks)
+        const uint64_t cost = (n * chunks + cus - 1u) / cus * s.vt * s.weight;
+        if (cost < least) {
+            least = cost;
+            best.vt = s.vt;
+        }
     }
-    const uint32_t nseq = a0.rows_per_seq ? a0.rows / a0.rows_per_seq : a0.rows;
-    hipLaunchKernelGGL(lmhead_fin, dim3(nseq), dim3(kLmThreads), 0, st, a0);
+    return best;
+}
+
+hipError_t launch_lmhead(const LmArgs& a0, uint32_t cus, hipStream_t st) {
+    LmArgs a = a0;
+    const LmShape sh = lmhead_shape(a.rows, a.vocab, a.hidden, cus);
+    const uint32_t cols = 64u * sh.vt;
+    a.nblocks = (a.vocab + cols - 1u) / cols;
+    a.nchunks = (a.rows + sh.br - 1u) / sh.br;
+    const dim3 grid(8u * ((a.nblocks + 7u) / 8u) * a.nchunks), block(kLmThreads);
+    // (stages: as deep as two workgroups a CU leave room for, or one where
+    // there is no second; two where two 256-column tiles a CU are all there
+    // is: 209 against 212 us)
+    if (a.hidden > kBigHidden) hipLaunchKernelGGL((lmhead_tile<4, 64, 3, true>), grid, block, 0, st, a);
+    else if (sh.br == 256u && sh.vt == 4u) hipLaunchKernelGGL((lmhead_tile<4, 256, 4>), grid, block, 0, st, a);
+    else if (sh.br == 256u) hipLaunchKernelGGL((lmhead_tile<2, 256, 3>), grid, block, 0, st, a);
+    else if (sh.br == 128u && sh.vt == 4u) hipLaunchKernelGGL((lmhead_tile<4, 128, 3>), grid, block, 0, st, a);
+    else if (sh.br == 128u) hipLaunchKernelGGL((lmhead_tile<2, 128, 4>), grid, block, 0, st, a);
+    else if (sh.vt == 5u) hipLaunchKernelGGL((lmhead_tile<5, 64, 3>), grid, block, 0, st, a);
+    else if (sh.vt == 4u && a.nblocks > cus && a.nblocks <= 2u * cus)
+        hipLaunchKernelGGL((lmhead_tile<4, 64, 2>), grid, block, 0, st, a);
+    else if (sh.vt == 4u) hipLaunchKernelGGL((lmhead_tile<4, 64, 4>), grid, block, 0, st, a);
+    else if (sh.vt == 2u) hipLaunchKernelGGL((lmhead_tile<2, 64, 4>), grid, block, 0, st, a);
+    else hipLaunchKernelGGL((lmhead_tile<1, 64, 6>), grid, block, 0, st, a);
+    const hipError_t e = hipGetLastError();
+    if (e != hipSuccess) return e;
+    const uint32_t nseq = a.rows_per_seq ? a.rows / a.rows_per_seq : a.rows;
+    constexpr uint32_t kMost = kLmMaxBlocks / kWave, kHalf = kMost / 2;
+    const bool half = a.nblocks <= kHalf * kWave;
+    if (a.rows_per_seq > 1u) {
+        if (half) hipLaunchKernelGGL((lmhead_fin<8, kHalf>), dim3(nseq), dim3(8 * kWave), 0, st, a);
+        else hipLaunchKernelGGL((lmhead_fin<8, kMost>), dim3(nseq), dim3(8 * kWave), 0, st, a);
+    } else {
+        if (half) hipLaunchKernelGGL((lmhead_fin<1, kHalf>), dim3(nseq), dim3(kWave), 0, st, a);
+        else hipLaunchKernelGGL((lmhead_fin<1, kMost>), dim3(nseq), dim3(kWave), 0, st, a);
+    }
     return hipGetLastError();
 }
 

@@ -113,6 +113,42 @@ def test_random_operands_within_the_f32_bound(sampler, rows, vocab, hidden):
     check_epilogue(g)
 
 
+# tiles of 64, 128 or 256 rows and 64 to 320 columns, with a row, a column and
+# a k-step more or less than full ones; the last: row offsets past 32 bits
+@pytest.mark.parametrize("rows,vocab,hidden", [
+    (3, 63, 64), (64, 129, 192), (63, 20001, 64), (64, 50257, 128), (2, 80001, 64), (17, 100001, 64),
+    (65, 255, 64), (128, 257, 128), (128, 50257, 64), (129, 256, 64), (255, 513, 192), (256, 50257, 64),
+    (257, 2049, 128), (300, 700, 320), (300, 50001, 64), (512, 512, 64), (3, 5, (1 << 22) + 64)])
+def test_row_tiles_are_exact(sampler, rows, vocab, hidden):
+    torch = sampler.torch
+    say("tiles", rows, vocab, hidden)
+    rng = np.random.default_rng(rows + vocab)
+    xi = rng.integers(-4, 5, (rows, hidden)).astype(np.float32)
+    wi = rng.integers(-3, 4, (vocab, hidden)).astype(np.float32)
+    ref = (xi.astype(np.int64) @ wi.astype(np.int64).T).astype(np.float32)
+    draft = rng.integers(0, vocab, rows).astype(np.int32)
+    draft[0], draft[rows - 1] = -1, vocab
+    d = torch.from_numpy(draft).cuda()
+    x, w = bf16(torch, xi).cuda(), bf16(torch, wi).cuda()
+    g = run(sampler, x, w, draft=d)
+    assert np.array_equal(g["logits"], ref)
+    check_epilogue(g)
+    # logprobs in f32 of values up to ~300: half a spacing beside the tolerance
+    lp = ref[np.arange(1, rows - 1), draft[1:-1]].astype(np.float64) - logsumexp64(ref)[1:-1]
+    assert (np.abs(g["draft_lp"][1:-1] - lp) <= LOGPROB_TOL + 0.5 * np.spacing(np.abs(lp).astype(np.float32))).all()
+    assert g["draft_lp"][0] == 0.0 and g["draft_lp"][rows - 1] == 0.0
+    # logits rows that are not 16-byte aligned, and no logits at all
+    big = torch.full((rows, vocab + 5), -7.0, dtype=torch.float32, device="cuda")
+    out = sampler.alloc_lmhead_out(rows, vocab, logits=False, draft=True)
+    sampler.lmhead_dev(x, w, dict(out, logits=big[:, 1:1 + vocab]), draft=d)
+    torch.cuda.synchronize()
+    assert np.array_equal(big[:, 1:1 + vocab].cpu().numpy(), ref)
+    assert (big[:, 0] == -7.0).all() and (big[:, 1 + vocab:] == -7.0).all()
+    h = run(sampler, x, w, draft=d, logits=False)
+    for k in ("argmax_ids", "log_z", "draft_lp"):
+        assert np.array_equal(h[k], g[k]) and np.array_equal(out[k].cpu().numpy(), g[k]), k
+
+
 @pytest.mark.parametrize("vocab", [20000, 140000])
 def test_drafts_and_acceptance(sampler, vocab):
     """rows_per_seq = 8: each sequence's drafts agree with the argmax on a
