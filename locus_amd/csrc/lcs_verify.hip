@@ -20,11 +20,13 @@
 
 namespace lcs {
 
-constexpr int kVerifyThreads = 256;
-
-template <int G>
-__global__ __launch_bounds__(kVerifyThreads) void verify_kernel(VerifyArgs a) {
-    constexpr int NT = kVerifyThreads;
+// NT: threads per row. A row's time is its rounds of NT x U 16-byte groups:
+// for few rows a memory latency and the round's arithmetic each (20 rows, V
+// 128256: 29.3 us a call with the running max moved per group and 256 threads,
+// 17.2 with it moved per round, 13.0 with 512 threads), for many the memory
+// stream (4096 bf16 rows, V 163840: 246 -> 234 us, 5.7 TB/s).
+template <int G, int NT>
+__global__ __launch_bounds__(NT) void verify_kernel(VerifyArgs a) {
     constexpr int U = 8;                   // 16-byte groups in flight per thread
     constexpr float kL2E = 1.4426950408889634f;
     __shared__ float redf[NT / kWave];
@@ -54,30 +56,36 @@ __global__ __launch_bounds__(kVerifyThreads) void verify_kernel(VerifyArgs a) {
             const uint32_t gi = g0 + u * NT + tid_x();
             r[u] = load16(rowp, gi < ng ? gi : 0u);
         }
+        // the round's group maxima first, so that the running max moves (and
+        // the sum is rescaled) at most once a round
+        float v[U][G], gm[U], m = NEG;
 #pragma unroll
         for (int u = 0; u < U; ++u) {
             const uint32_t gi = g0 + u * NT + tid_x();
-            if (gi >= ng) continue;
-            float v[G];
-            decode<G>(r[u], v);
-            if (gi * G + G > V) {
+            decode<G>(r[u], v[u]);
+            if ((g0 + (u + 1) * NT) * G > V) {   // (uniform: the row's last groups)
 #pragma unroll
-                for (int k = 0; k < G; ++k) v[k] = gi * G + k < V ? v[k] : NEG;
+                for (int k = 0; k < G; ++k) v[u][k] = gi * G + k < V ? v[u][k] : NEG;
             }
-            float gm = v[0];
+            gm[u] = v[u][0];
 #pragma unroll
-            for (int k = 1; k < G; ++k) gm = fmaxf(gm, v[k]);
-            if (gm > om) {
-                os = om == NEG ? 0.0 : os * (double)__builtin_amdgcn_exp2f((om - gm) * kL2E);
-                om = gm;
-                bg = gi;
-                b = -om * kL2E;
-                corr = (double)__builtin_amdgcn_exp2f(-fmaf(om, kL2E, b));
-            }
-            if (om != NEG) {
+            for (int k = 1; k < G; ++k) gm[u] = fmaxf(gm[u], v[u][k]);
+            m = fmaxf(m, gm[u]);
+        }
+        if (m > om) {
+            os = om == NEG ? 0.0 : os * (double)__builtin_amdgcn_exp2f((om - m) * kL2E);
+            om = m;
+#pragma unroll
+            for (int u = U - 1; u >= 0; --u) bg = gm[u] == m ? g0 + u * NT + tid_x() : bg;
+            b = -om * kL2E;
+            corr = (double)__builtin_amdgcn_exp2f(-fmaf(om, kL2E, b));
+        }
+        if (om != NEG) {
+#pragma unroll
+            for (int u = 0; u < U; ++u) {
                 float c[G];
 #pragma unroll
-                for (int k = 0; k < G; ++k) c[k] = __builtin_amdgcn_exp2f(fmaf(v[k], kL2E, b));
+                for (int k = 0; k < G; ++k) c[k] = __builtin_amdgcn_exp2f(fmaf(v[u][k], kL2E, b));
 #pragma unroll
                 for (int w = G / 2; w >= 1; w /= 2)
 #pragma unroll
@@ -111,26 +119,40 @@ __global__ __launch_bounds__(kVerifyThreads) void verify_kernel(VerifyArgs a) {
 }
 
 // Acceptance length per sequence (engine.cpp:366-383): leading rows whose
-// argmax equals their draft. One thread per sequence.
-__global__ __launch_bounds__(256) void accept_kernel(VerifyArgs a) {
-    const uint32_t seq = wg_x() * 256u + tid_x();
+// argmax equals their draft. A wave per sequence, a row per lane (rows_per_seq
+// <= 64): one memory round trip instead of one per accepted row.
+constexpr uint32_t kAcceptSeqs = 4;   // sequences per workgroup
+__global__ __launch_bounds__(kAcceptSeqs * kWave) void accept_kernel(VerifyArgs a) {
+    const uint32_t seq = wg_x() * kAcceptSeqs + tid_x() / kWave;
     if (seq >= a.n_seq) return;
-    const uint32_t base = seq * a.rows_per_seq;
-    uint32_t acc = 0;
-    while (acc < a.rows_per_seq && a.argmax_ids[base + acc] == a.draft[base + acc]) ++acc;
-    a.accept_len[seq] = acc;
+    const uint32_t lane = (uint32_t)lane_id(), R = a.rows_per_seq;
+    const uint32_t row = seq * R + (lane < R ? lane : 0u);
+    const uint64_t miss = ballot(lane >= R || a.argmax_ids[row] != a.draft[row]);
+    const uint32_t acc = miss ? min((uint32_t)__builtin_ctzll(miss), R) : R;
+    if (lane == 0u) a.accept_len[seq] = acc;
+}
+
+// Threads per row: a row of more than two rounds of 512 threads takes 512 (us
+// a call with 256 / 512 / 1024 threads, f32, V 128256: 20 rows 17.2 / 13.0 /
+// 13.0, 128 rows 19.6 / 15.6 / 17.2, 2048 rows 187.5 / 187.1 / 189; bf16, V
+// 163840, 4096 rows 238.3 / 233.8 / 267), except where about two rows a CU
+// make one uneven round of the larger workgroups (512 rows: 51.4 / 52.7, bf16
+// 34.9 / 36.6). A shorter row leaves them idle (2048 rows of V 5000: 13.3 /
+// 17.1).
+template <int G>
+static void launch_rows(const VerifyArgs& a, hipStream_t st) {
+    const uint32_t rows = a.n_seq * a.rows_per_seq;
+    const bool wide = (a.vocab + G - 1u) / G > 8192u && (rows <= 256u || rows > 768u);
+    if (wide) hipLaunchKernelGGL((verify_kernel<G, 512>), dim3(rows), dim3(512), 0, st, a);
+    else hipLaunchKernelGGL((verify_kernel<G, 256>), dim3(rows), dim3(256), 0, st, a);
 }
 
 hipError_t launch_verify(const VerifyArgs& a, hipStream_t st) {
-    const dim3 grid(a.n_seq * a.rows_per_seq), block(kVerifyThreads);
-    if (a.dtype == LCS_BF16) {
-        hipLaunchKernelGGL(verify_kernel<8>, grid, block, 0, st, a);
-    } else {
-        hipLaunchKernelGGL(verify_kernel<4>, grid, block, 0, st, a);
-    }
-    hipError_t e = hipGetLastError();
+    if (a.dtype == LCS_BF16) launch_rows<8>(a, st);
+    else launch_rows<4>(a, st);
+    const hipError_t e = hipGetLastError();
     if (e != hipSuccess) return e;
-    hipLaunchKernelGGL(accept_kernel, dim3((a.n_seq + 255u) / 256u), dim3(256), 0, st, a);
+    hipLaunchKernelGGL(accept_kernel, dim3((a.n_seq + kAcceptSeqs - 1u) / kAcceptSeqs), dim3(kAcceptSeqs * kWave), 0, st, a);
     return hipGetLastError();
 }
 

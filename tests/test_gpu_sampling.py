@@ -693,3 +693,37 @@ def test_top_n_with_clustered_maxima(sampler):
                        base.hist_off, base.hist_ids, None, n_top, True)
         g = run(sampler, w)
         compare(w, g, O.sample_batch(w, threads=8), w.name, expect_paths={2, 3, 4})
+
+
+@pytest.mark.parametrize("V,dtype,n_seq,per", [(32765, "f32", 3, 5), (32772, "f32", 3, 64), (65529, "bf16", 1, 1),
+                                               (65536, "bf16", 2, 7), (65545, "bf16", 5, 2), (40001, "f32", 60, 5),
+                                               (9, "f32", 7, 3)])
+def test_verify_workgroup_sizes(sampler, V, dtype, n_seq, per):
+    """Both workgroup sizes of the verify kernel at the edges of their rounds:
+    rows that end inside a group, the maximum in the first or last group, in
+    two groups (the first index wins), rows of one value and of -inf."""
+    rows = n_seq * per
+    g = np.random.default_rng([V, rows])
+    x = (g.standard_normal((rows, V), dtype=np.float32) * 2).astype(np.float32)
+    x[0, V - 1] = 40.0
+    if rows > 4:
+        x[1, 0] = 40.0
+        x[2, [V // 2, V - 1]] = 40.0
+        x[3] = 1.0
+        x[4, 1:] = -np.inf
+    logits = W.bf16_rne(x) if dtype == "bf16" else x
+    f = W.bf16_to_f32(logits) if dtype == "bf16" else x
+    am = f.argmax(1).astype(np.int32)
+    draft = np.where(g.random(rows) < 0.8, am, g.integers(0, V, rows)).astype(np.int32)
+    w = W.Workload("verify", rows, V, dtype, logits, None, None, None, n_seq=n_seq, rows_per_seq=per, draft=draft)
+    got = sampler.verify(w)
+    assert np.array_equal(got["argmax_ids"], am)
+    ok = (am == draft).reshape(n_seq, per)
+    assert got["accept_len"].tolist() == [int(np.cumprod(r).sum()) for r in ok]
+    m = f.max(1).astype(np.float64)
+    lz = m + np.log(np.exp(f.astype(np.float64) - m[:, None]).sum(1))
+    lp = f[np.arange(rows), draft].astype(np.float64) - lz
+    fin = np.isfinite(lp)
+    # (logprobs of up to ~45 in f32: half a spacing beside the tolerance)
+    assert (np.abs(got["draft_lp"][fin] - lp[fin]) <= 1e-6 + 0.5 * np.spacing(np.abs(lp[fin]).astype(np.float32))).all()
+    assert np.array_equal(got["draft_lp"][~fin], lp[~fin].astype(np.float32))
