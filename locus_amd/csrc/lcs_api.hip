@@ -5,6 +5,7 @@
 #include <hip/hip_runtime.h>
 
 #include <atomic>
+#include <cmath>
 #include <cstdio>
 #include <cstring>
 #include <mutex>
@@ -207,6 +208,24 @@ __global__ void clear_words(uint32_t* w, uint32_t n) {
     for (uint32_t i = threadIdx.x; i < n; i += blockDim.x) w[i] = 0u;
 }
 
+// Whether a batch holds min-p window rows that may well overflow: the cut lies
+// T ln(1 / min_p) logits below the maximum (T 0.7, min-p 0.05: 2.1; T 1, 0.01:
+// 4.6; T 1.5, 0.05: 4.5). With logits of spread 2 to 3, a cut 4 below the
+// maximum of V 128256 leaves more than the 64 ids a slice's record holds. One
+// row that overflows costs the call 450-500 us in row_fin's exact path, the
+// five nucleus launches 9-10 us where no row does (V 128256, us a call without
+// / with them: flat rows, 1 row 516 / 84, 64 rows 544 / 117; confident rows, 1
+// row 16.0 / 25.2, 64 rows 22.5 / 32.9).
+constexpr float kWideWindow = 4.0f;
+bool wide_windows(const lcs_batch* b) {
+    for (uint32_t r = 0; r < b->rows; ++r) {
+        const lcs_params& p = b->params_host[r];
+        if (lcs::row_mode(p, false, b->vocab) == lcs::kModeWindow && p.temperature * -std::log(p.min_p) >= kWideWindow)
+            return true;
+    }
+    return false;
+}
+
 // lcs_sample on the workspace of c (a context, or the no-alloc entry's view
 // of its static array); validation first, nothing is launched on an error.
 // clear_status: the status word is zeroed ahead of the kernels.
@@ -278,6 +297,10 @@ int sample_impl(lcs_ctx* c, const lcs_batch* b, const lcs_out* o, void* stream, 
             }
         }
     }
+    // Window rows whose min-p cut lies far below the maximum (T ln(1 / min_p)
+    // logits) often overflow their slices' window records; the nucleus
+    // kernels are then launched after the sliced ones to take those that do.
+    const bool wide = any_slice && !b->win_slot && b->params_host && wide_windows(b);
     if (b->flags & LCS_WRITE_PENALIZED) { any_slice = false; any_nucleus = false; any_general = true; }
 
     lcs::SampleArgs a{};
@@ -286,7 +309,7 @@ int sample_impl(lcs_ctx* c, const lcs_batch* b, const lcs_out* o, void* stream, 
     a.rows = b->rows;
     a.vocab = b->vocab;
     a.dtype = b->dtype;
-    a.flags = b->flags;
+    a.flags = b->flags & (LCS_WANT_LOGPROBS | LCS_WRITE_PENALIZED);
     a.n_top = want_lp ? b->n_top : 0;
     a.mask_words = b->mask_words;
     a.params = b->params;
@@ -318,6 +341,8 @@ int sample_impl(lcs_ctx* c, const lcs_batch* b, const lcs_out* o, void* stream, 
     a.ss_modes = ss_modes;
     // likewise for the nucleus kernels when every row takes that path
     a.all_nucleus = (b->params_host && !any_general && !any_slice) ? 1u : 0u;
+    const bool run_nucleus = any_nucleus || (wide && any_slice);
+    if (any_slice && run_nucleus && !b->win_slot) a.flags |= lcs::kFlagNucAfter;
     a.nrow = c->nrow;
     a.nh_pk = c->nh_pk;
     a.nlist = c->nlist;
@@ -340,7 +365,7 @@ int sample_impl(lcs_ctx* c, const lcs_batch* b, const lcs_out* o, void* stream, 
     }
     if (any_general && (e = lcs::launch_general(a, st)) != hipSuccess) return hip_fail(c, e, "general kernel launch");
     if (any_slice && (e = lcs::launch_slice(a, st)) != hipSuccess) return hip_fail(c, e, "slice kernel launch");
-    if (any_nucleus && (e = lcs::launch_nucleus(a, st)) != hipSuccess) return hip_fail(c, e, "nucleus kernels launch");
+    if (run_nucleus && (e = lcs::launch_nucleus(a, st)) != hipSuccess) return hip_fail(c, e, "nucleus kernels launch");
     return LCS_OK;
 }
 

@@ -690,6 +690,7 @@ __device__ __forceinline__ void fin_row(const lcs_params* params, const uint64_t
     }
     PROF_AT(kProfFin + row, 20 + wv);
     const bool stoch = mode == kModeWindow, topk = mode == kModeTopK;
+    if ((flags & kFlagNucAfter) != 0u && stoch && tid == 0) const_cast<uint64_t*>(srecs)[wide_flag_at(row)] = 0ull;
     const float inv_t = stoch || topk ? fdiv(1.0f, P.temperature) : 1.0f;
     const double u = (stoch || topk) && wv == 0 ? a.u[row] : 0.0;
     PROF_AT(kProfFin + row, 4 + wv);
@@ -760,7 +761,18 @@ __device__ __forceinline__ void fin_row(const lcs_params* params, const uint64_t
         __syncthreads();
         if (!sm.fin_fb_decide) return;
     }
-    // the records cannot settle this row: the exact single-workgroup path
+    // the records cannot settle this row. When the nucleus kernels follow,
+    // they take it with all its slices (64 rows of V 128256 whose windows hold
+    // thousands of ids: 117 us a call against 541 with exact_row's one workgroup a
+    // row); a penalty window above max_hist stays here, where it is reported
+    if ((flags & kFlagNucAfter) != 0u && stoch && !(want_lp && sm.fin_fb[1] != 0u)) {
+        const uint32_t hn = penalties_active(P) && a.hist_off != nullptr ? a.hist_off[row + 1] - a.hist_off[row] : 0u;
+        if (min(hn, P.repeat_last_n) <= a.max_hist) {   // (uniform)
+            if (tid == 0) const_cast<uint64_t*>(srecs)[wide_flag_at(row)] = 1ull;
+            return;
+        }
+    }
+    // else the exact single-workgroup path
     // (out of line: it reads the kernel arguments from an LDS copy). Unless
     // the log-normaliser's wave flagged the row, the records still give its
     // penalised maximum and log-normaliser (and the top-n is written), and

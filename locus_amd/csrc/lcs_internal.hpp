@@ -53,6 +53,16 @@ constexpr uint32_t kFlagPenOverflow = 8u;          // more penalised groups than
 constexpr uint32_t kFlagExact = 16u;               // the row is resolved on the exact path
 }  // namespace rec
 
+// SampleArgs::flags: the nucleus kernels follow the sliced ones in this call and
+// take the window rows that their records cannot settle (row_fin sets the word
+// of such a row's first record at wide_flag_at). A flag bit, since the kernels
+// have the flags in registers from the start.
+constexpr uint32_t kFlagNucAfter = 1u << 31;
+__host__ __device__ inline uint64_t wide_flag_at(uint32_t row) {
+    static_assert(rec::kWinRaw + kWinCap < rec::kWords64, "a spare word");
+    return ((uint64_t)row * kRecsPerRow + 1u) * rec::kWords64 - 1u;
+}
+
 // ---- single-workgroup exact path ----
 constexpr int kGenThreads = 1024;
 constexpr uint32_t kGenBins = 2048;
@@ -97,6 +107,7 @@ constexpr uint32_t kNucRanges = 4;      // bin ranges a row's decisions can need
 constexpr uint32_t kNucSub = 128;       // sub-bins per range in the select pass
 constexpr float kNucXFloor = -128.0f;   // offsets below collapse into the last bin
 constexpr uint32_t kNucFallback = 1u;   // row state flag: resolve with exact_row
+constexpr uint32_t kNucOff = 2u;        // row state flag: penalised candidates may lie past the bins
 struct NucRange {
     uint32_t b0, b1;   // bins [b0, b1]
     uint32_t c0, cnt;  // candidates before the range, in it

@@ -71,7 +71,7 @@ struct NucLocal {
     float piv[4];                   // or, for at most two ranges, their logit intervals (select pass)
     float mraw[kNW];
     double sraw[kNW];
-    float mpen[kNW], npen[kNW], mmsk[kNW], nmsk[kNW];
+    float mpen[kNW], npen[kNW], mmsk[kNW], nmsk[kNW], nraw[kNW];
     uint32_t ipen[kNW], imsk[kNW], nall[kNW];
     uint64_t ck[kNucCand];
     // select-pass finalize
@@ -83,7 +83,7 @@ struct NucLocal {
     uint32_t out_flag;
     // the row state pass B's workgroups derive from pass A's records
     float st_maxl, st_sx;
-    uint32_t st_use_mask, st_fallback;
+    uint32_t st_use_mask, st_fallback, st_off;
     NucRange rgl[kNucRanges];  // the planned ranges, for lookups by a computed index (select finalize)
     SampleArgs args;           // for the exact fallback
 };
@@ -382,6 +382,14 @@ __device__ __forceinline__ void nuc_taylor(float sx, double scale, bool minus_on
     }
 }
 
+// Whether the nucleus kernels serve a row: one of their own, or a window row
+// that row_fin handed over in this call.
+__device__ __forceinline__ bool nuc_takes(const SampleArgs& a, uint32_t row, const lcs_params& P, bool masked) {
+    const uint32_t mode = row_mode(P, masked, a.vocab);
+    if (mode == kModeNucleus) return true;
+    return mode == kModeWindow && (a.flags & kFlagNucAfter) != 0u && scalar_load(a.srecs + wide_flag_at(row)) != 0ull;
+}
+
 // Row and mode of a finalize workgroup (one per row of the launch); false
 // when the row is not on the nucleus path.
 __device__ __forceinline__ bool nuc_fin_row(const SampleArgs& a, uint32_t& row, lcs_params& P, bool& masked) {
@@ -389,7 +397,7 @@ __device__ __forceinline__ bool nuc_fin_row(const SampleArgs& a, uint32_t& row, 
     if (row >= a.rows) return false;
     P = scalar_load(a.params + row);
     masked = a.mask != nullptr && (a.has_mask == nullptr || scalar_load_u8(a.has_mask + row) != 0);
-    return row_mode(P, masked, a.vocab) == kModeNucleus;
+    return nuc_takes(a, row, P, masked);
 }
 
 // Row and mode for a nucleus launch; false when this workgroup has no work.
@@ -401,7 +409,7 @@ __device__ __forceinline__ bool nuc_row(const SampleArgs& a, uint32_t& row, uint
     if (row >= a.rows || wg_x() / S >= kNucRows) return false;
     P = scalar_load(a.params + row);
     masked = a.mask != nullptr && (a.has_mask == nullptr || scalar_load_u8(a.has_mask + row) != 0);
-    return row_mode(P, masked, a.vocab) == kModeNucleus;
+    return nuc_takes(a, row, P, masked);
 }
 
 // Kernel arguments the nucleus kernels take ahead of SampleArgs: the build
@@ -430,7 +438,10 @@ constexpr uint32_t kHdr = 8;
 // 1: f64 sum exp(raw - raw max)
 // 2: f32 penalised max | u32 its index       3: same over allowed ids
 // 4: u32 allowed ids                          5: f32 penalised min | f32 allowed min
+// 6: f32 raw min of the candidates (the allowed ids of a constrained row) in a row with penalties, else -inf
 constexpr uint32_t kTop = kHdr;               // kTopMax rank keys, ascending
+constexpr uint32_t kOff = kTop + kTopMax;     // pass B: f64 mass of the candidates past the bins, then their u64 count
+static_assert(kOff + 2 <= rec::kWords64, "record size");
 }  // namespace nrec
 
 template <int G>
@@ -516,8 +527,18 @@ __global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(4))) void nu
             }
         }
     }
-    if (in.hany) in.apply(sm);
     in.finish_mask();
+    if (in.hany) {
+        // rows with penalties: the raw candidates' min (the bins need not
+        // reach the penalised ones below it)
+        float nr = __builtin_huge_valf();
+        const uint32_t cm = in.cand_bits(in.mrow != nullptr);
+#pragma unroll
+        for (int q = 0; q < kSliceElems; ++q) nr = ((cm >> q) & 1u) ? fminf(nr, in.v[q]) : nr;
+        nr = wave_min(nr);
+        if (lane == 0) sm.l.nraw[wv] = nr;
+        in.apply(sm);
+    }
     // penalised candidate statistics over all ids and over the allowed ids
     {
         float bv = NEG, mv = NEG, nb = __builtin_huge_valf(), nm = __builtin_huge_valf();
@@ -567,6 +588,7 @@ __global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(4))) void nu
         const float na_ = __builtin_huge_valf();
         const float mnb = wave_min(lw ? sm.l.npen[wl] : na_);
         const float mnm = wave_min(lw ? sm.l.nmsk[wl] : na_);
+        const float mnr = in.hany ? wave_min(lw ? sm.l.nraw[wl] : na_) : -na_;   // (-inf: not known)
         wave_argmax(ma, ia);
         wave_argmax(mm, im);
         const uint32_t na = wave_sum_u(lw ? sm.l.nall[wl] : 0u);
@@ -580,9 +602,10 @@ __global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(4))) void nu
             case 3: hw = pack2(__float_as_uint(mm), im); break;
             case 4: hw = (uint64_t)na; break;
             case 5: hw = pack2(__float_as_uint(mnb), __float_as_uint(mnm)); break;
+            case 6: hw = __float_as_uint(mnr); break;
             default: break;
         }
-        if (lane < 6) myrec[lane] = hw;
+        if (lane < 7) myrec[lane] = hw;
     } else if (wv == 1) {
         const uint32_t nts = min(ntop, in.len);
         const uint32_t ncc = min(sm.l.ncand, kNucCand);
@@ -610,6 +633,7 @@ struct NucState {
     float maxl, sx;
     uint32_t maxi, n_cand;
     bool use_mask, fallback;
+    bool off;   // penalised candidates lie past the bins
 };
 __device__ __forceinline__ NucState nuc_row_state(const SampleArgs& a, uint32_t row, const lcs_params& P,
                                                   bool masked, uint32_t ntop) {
@@ -619,7 +643,7 @@ __device__ __forceinline__ NucState nuc_row_state(const SampleArgs& a, uint32_t 
     const uint64_t* recs = reinterpret_cast<const uint64_t*>(a.recs) + (uint64_t)row * S * rec::kWords64;
     const bool mine = (uint32_t)lane < S;
     const uint64_t* my = recs + (mine ? lane : 0) * rec::kWords64;
-    const uint64_t h0 = my[0], h2 = my[2], h3 = my[3], h4 = my[4], h5 = my[5];
+    const uint64_t h0 = my[0], h2 = my[2], h3 = my[3], h4 = my[4], h5 = my[5], h6 = my[6];
     const bool ovf = ntop && ballot(mine && ((uint32_t)(h0 >> 48) & rec::kFlagCandOverflow));
     const uint32_t na = wave_sum_u(mine ? (uint32_t)h4 : 0u);
     const bool use_mask = masked && na > 0;
@@ -631,6 +655,17 @@ __device__ __forceinline__ NucState nuc_row_state(const SampleArgs& a, uint32_t 
                                    : __builtin_huge_valf());
     const float inv_t = fdiv(1.0f, P.temperature);
     float x_lo = (mx == NEG) ? 0.0f : tempered(mn, mx, inv_t);
+    // Penalties push a few ids far down (frequency 0.5 x a count of 200), and
+    // bins that reach them would be too coarse where the mass is: the bins
+    // reach the raw candidates' min, what lies below it (at most the penalty
+    // window's ids) is summed apart. (A mask that allows nothing: its raw min
+    // is +inf, not used.)
+    const float rn = wave_min(mine ? __uint_as_float((uint32_t)h6) : __builtin_huge_valf());
+    bool off = false;
+    if (rn > mn && rn <= mx && tempered(rn, mx, inv_t) >= kNucXFloor) {
+        x_lo = tempered(rn, mx, inv_t);
+        off = true;   // (mn is past the bins, or at least may be)
+    }
     if (!(x_lo >= kNucXFloor)) x_lo = kNucXFloor;   // also NaN
     // bins per unit offset: the largest power of two in [4, 2^20] with
     // kNucBins / sx >= -x_lo
@@ -646,6 +681,7 @@ __device__ __forceinline__ NucState nuc_row_state(const SampleArgs& a, uint32_t 
     st.n_cand = use_mask ? na : a.vocab;
     st.use_mask = use_mask;
     st.fallback = ovf;
+    st.off = off;
     return st;
 }
 
@@ -726,13 +762,14 @@ __global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(4))) void nu
             sm.l.st_sx = st.sx;
             sm.l.st_use_mask = st.use_mask ? 1u : 0u;
             sm.l.st_fallback = st.fallback ? 1u : 0u;
+            sm.l.st_off = st.off ? 1u : 0u;
             if (slice == 0) {
                 nr->maxl = st.maxl;
                 nr->maxi = st.maxi;
                 nr->sx = st.sx;
                 nr->n_cand = st.n_cand;
                 nr->use_mask = st.use_mask ? 1u : 0u;
-                nr->flags = st.fallback ? kNucFallback : 0u;
+                nr->flags = (st.fallback ? kNucFallback : 0u) | (st.off ? kNucOff : 0u);
                 nr->nr = 0u;
                 nr->list_n = 0u;
             }
@@ -768,16 +805,21 @@ __global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(4))) void nu
     // 2^-37 / sx relative to a candidate's weight (1.8e-12 at sx = 4), far
     // under the plan's 1e-10 guard.
     //
-    // Candidates past the grid (f > kNucBins, only when x_lo was floored at
-    // -128, so sx = 4 and x < -128) count in the last bin with r clamped to
-    // -1: mass below e^-128 each, also far under the guard. A wave skips an
+    // Candidates past the grid (f > kNucBins) count in the last bin. Where
+    // x_lo was floored at -128 (sx = 4 and x < -128) with r clamped to -1: mass
+    // below e^-128 each, also far under the guard. In a row whose bins end at
+    // the raw candidates' min (st.off) with r = 0's word (v = 0), and their
+    // mass exp_f64(x) and number go to the slice's record; the finalize puts
+    // the last bin's mass right. A wave skips an
     // element position none of its lanes holds a candidate at (sparse
     // constraint masks); a wave whose lanes hold only candidates tests none.
     if (masked) in.finish_mask();
     const uint32_t cm = in.cand_bits(use_mask);
     const bool all_cand = ballot(cm != 0xffffffffu) == 0u;
     const double two_k = 68719476736.0 * (double)sx;   // 2^36 sx
-    auto fill = [&](auto deg, auto all) {
+    double off_m = 0.0;
+    uint32_t off_n = 0u;
+    auto fill = [&](auto deg, auto all, auto past) {
         constexpr int n = decltype(deg)::value;
         constexpr bool off_grid = n == 8;   // (only when sx = 4: f may pass kNucBins)
         double q[n + 1];   // (exp(d) - 1) 2^k
@@ -793,7 +835,12 @@ __global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(4))) void nu
 #pragma unroll
                 for (int j = n - 1; j >= 0; --j) p = __builtin_fma(p, r, q[j]);
                 const double y = p + 0x1.8p52;   // rint(p) + 1.5 * 2^52, exactly
-                const uint64_t w = (uint64_t)__double_as_longlong(y) + (kPkOne - kPkMagic);
+                uint64_t w = (uint64_t)__double_as_longlong(y) + (kPkOne - kPkMagic);
+                if (decltype(past)::value && f > (float)kNucBins) {
+                    w = kPkOne;
+                    off_m += exp_f64((double)x);
+                    off_n += 1u;
+                }
                 atomicAdd(reinterpret_cast<unsigned long long*>(&g_nuc.u.pk[(uint32_t)fb]), (unsigned long long)w);
             }
         }
@@ -801,17 +848,28 @@ __global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(4))) void nu
     using D5 = std::integral_constant<int, 5>;
     using D6 = std::integral_constant<int, 6>;
     using D8 = std::integral_constant<int, 8>;
-    using All = std::true_type;
-    using Some = std::false_type;
-    if (sx >= 64.0f) {
-        if (all_cand) fill(D5{}, All{});
-        else fill(D5{}, Some{});
+    using Yes = std::true_type;
+    using No = std::false_type;
+    if (sm.l.st_off) {
+        if (sx >= 64.0f) fill(D5{}, No{}, Yes{});
+        else if (sx >= 16.0f) fill(D6{}, No{}, Yes{});
+        else fill(D8{}, No{}, Yes{});
+        off_m = block_sum<NT>(off_m, sm.l.sraw);
+        off_n = block_sum_u<NT>(off_n, sm.l.nall);
+        if (tid == 0) {
+            uint64_t* orec = reinterpret_cast<uint64_t*>(a.recs) + ((uint64_t)row * a.slices + slice) * rec::kWords64 + nrec::kOff;
+            orec[0] = d_bits(off_m);
+            orec[1] = off_n;
+        }
+    } else if (sx >= 64.0f) {
+        if (all_cand) fill(D5{}, Yes{}, No{});
+        else fill(D5{}, No{}, No{});
     } else if (sx >= 16.0f) {
-        if (all_cand) fill(D6{}, All{});
-        else fill(D6{}, Some{});
+        if (all_cand) fill(D6{}, Yes{}, No{});
+        else fill(D6{}, No{}, No{});
     } else {
-        if (all_cand) fill(D8{}, All{});
-        else fill(D8{}, Some{});
+        if (all_cand) fill(D8{}, Yes{}, No{});
+        else fill(D8{}, No{}, No{});
     }
     __syncthreads();
     uint64_t* gp = a.nh_pk + ((uint64_t)wrow * kMaxSlices + slice) * kNucBins;
@@ -874,10 +932,23 @@ __global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(1, 2))) void
             }
         }
         const double inv_2k = 1.0 / (68719476736.0 * (double)sx);
+        // the candidates past the bins (the last bin's thread): their number
+        // out of its count for the mass, their own mass in
+        double off_m = 0.0;
+        uint32_t off_n = 0u;
+        if ((nr->flags & kNucOff) && tid == NT - 1) {
+            const uint64_t* orec = reinterpret_cast<const uint64_t*>(a.recs) + (uint64_t)row * S * rec::kWords64 + nrec::kOff;
+            for (uint32_t ss = 0; ss < S; ++ss) {
+                off_m += bits_d(orec[(uint64_t)ss * rec::kWords64]);
+                off_n += (uint32_t)orec[(uint64_t)ss * rec::kWords64 + 1];
+            }
+        }
 #pragma unroll
         for (uint32_t k = 0; k < BPT; ++k) {
+            if (k == BPT - 1) vs[k] -= (int64_t)((double)off_n * (68719476736.0 * (double)sx));   // (an integer)
             m[k] = ((double)c[k] + (double)vs[k] * inv_2k) * exp_f64(-((double)(tid * BPT + k) + 0.5) * inv_sx);
         }
+        m[BPT - 1] += off_m;
     }
     NPROF(row, 1);
     {
@@ -1024,7 +1095,9 @@ __global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(1, 2))) void
     nr->nr = nm_;
     nr->list_n = 0u;
     NPROF(row, 3);
-    if (total > kNucList || ncand != ncand_row) nr->flags |= kNucFallback;
+    // (a decision among candidates past the bins has no sub-bins to go by)
+    const bool past = (nr->flags & kNucOff) && cur_b < NB && cur_e == NB - 1;
+    if (total > kNucList || ncand != ncand_row || past) nr->flags |= kNucFallback;
 }
 
 // ========================================================= C: nuc_select ==
@@ -1617,7 +1690,8 @@ __device__ __forceinline__ bool nuc_select_fin(const SampleArgs& a, uint32_t row
             dg.keep = keep;
             dg.maxl = maxl;
             dg.boundary = last_key != ~0ull ? rank_val(last_key) : maxl;
-            dg.path = LCS_PATH_NUCLEUS;
+            // (a window row handed over is an exact fallback to the caller)
+            dg.path = row_mode(P, false, a.vocab) == kModeWindow ? LCS_PATH_GENERAL : LCS_PATH_NUCLEUS;
             dg.sum = SK;
             dg.kept_sum = kept_sum;
             a.diag[row] = dg;
