@@ -23,6 +23,7 @@ hipError_t launch_win_load(WinHdr* wh, int32_t* wring, uint64_t* wbkt, uint32_t 
 hipError_t launch_general(const SampleArgs& a, hipStream_t st);
 hipError_t launch_nucleus(const SampleArgs& a, hipStream_t st);
 hipError_t launch_verify(const VerifyArgs& a, hipStream_t st);
+hipError_t launch_logprobs(const LogprobArgs& a, uint32_t dtype, hipStream_t st);
 hipError_t launch_draft(const DraftArgs& a, hipStream_t st);
 hipError_t launch_lmhead(const LmArgs& a, uint32_t cus, hipStream_t st);
 uint32_t lmhead_max_blocks(uint32_t vocab, uint32_t cus);
@@ -208,6 +209,25 @@ __global__ void clear_words(uint32_t* w, uint32_t n) {
     for (uint32_t i = threadIdx.x; i < n; i += blockDim.x) w[i] = 0u;
 }
 
+// Whether a batch with logprobs is greedy rows without penalties or a mask
+// (lcs_logprobs, or lcs_sample as such) that the one-kernel path serves: a
+// workgroup per row streams it once. Below 64 rows a long row is faster cut
+// into slices (us, sliced / whole: V 128256 bf16, 16 rows 11.2 / 12.0, 64 rows
+// 13.9 / 12.5, 1024 rows 99.8 / 55.1; f32 11.0 / 12.7, 14.8 / 14.5, 113.6 /
+// 101.1); up to 8192 16-byte groups the second launch costs more than the
+// slices save (V 32000, 16 rows 11.1 / 7.7).
+bool plain_greedy(const lcs_batch* b, const lcs_out* o) {
+    if (!b->params_host || b->mask || b->raw_stats || o->diag || b->win_slot || (b->flags & LCS_WRITE_PENALIZED)) return false;
+    const uint32_t g = b->dtype == LCS_BF16 ? 8u : 4u;
+    if (b->rows < 64u && (b->vocab + g - 1u) / g > 8192u) return false;
+    for (uint32_t r = 0; r < b->rows; ++r) {
+        const lcs_params& p = b->params_host[r];
+        const bool pen = !(p.repeat_penalty == 1.0f && p.frequency_penalty == 0.0f && p.presence_penalty == 0.0f);
+        if (!(p.temperature <= 0.0f) || (pen && b->hist_off)) return false;
+    }
+    return true;
+}
+
 // Whether a batch holds min-p window rows that may well overflow: the cut lies
 // T ln(1 / min_p) logits below the maximum (T 0.7, min-p 0.05: 2.1; T 1, 0.01:
 // 4.6; T 1.5, 0.05: 4.5). With logits of spread 2 to 3, a cut 4 below the
@@ -275,6 +295,22 @@ int sample_impl(lcs_ctx* c, const lcs_batch* b, const lcs_out* o, void* stream, 
         for (uint32_t r = 0; r < b->rows; ++r) {
             if (b->params_host[r].temperature > 0.0f) return fail(c, LCS_ERR_INVALID_ARG, "u missing for a stochastic row");
         }
+    }
+    if (want_lp && !clear_status && plain_greedy(b, o)) {
+        lcs::LogprobArgs a{};
+        a.logits = b->logits;
+        a.row_stride = b->row_stride;
+        a.rows = b->rows;
+        a.vocab = b->vocab;
+        a.n_top = b->n_top;
+        a.chosen = b->lp_ids;
+        a.ids = o->ids;
+        a.chosen_lp = o->chosen_lp;
+        a.top_ids = o->top_ids;
+        a.top_lp = o->top_lp;
+        DeviceGuard g(c->device);
+        const hipError_t e = lcs::launch_logprobs(a, b->dtype, static_cast<hipStream_t>(stream));
+        return e == hipSuccess ? LCS_OK : hip_fail(c, e, "logprobs kernel launch");
     }
     // Which kernels to launch: a row runs in exactly one of them (the
     // kernels re-derive each row's mode on the device). Without a host copy

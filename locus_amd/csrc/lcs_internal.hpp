@@ -216,6 +216,18 @@ struct VerifyArgs {
     uint32_t* accept_len;
 };
 
+// lcs_logprobs over many rows (lcs_verify.hip)
+struct LogprobArgs {
+    const void* logits;
+    uint64_t row_stride;
+    uint32_t rows, vocab, n_top;
+    const int32_t* chosen;          // rows, or NULL: each row's argmax
+    int32_t* ids;                   // rows, or NULL
+    float* chosen_lp;
+    int32_t* top_ids;
+    float* top_lp;
+};
+
 // n-gram drafts (lcs_draft.hip)
 constexpr uint32_t kDraftMaxNgram = 64;
 constexpr uint32_t kDraftMaxLen = 256;

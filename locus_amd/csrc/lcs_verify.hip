@@ -20,31 +20,28 @@
 
 namespace lcs {
 
-// NT: threads per row. A row's time is its rounds of NT x U 16-byte groups:
-// for few rows a memory latency and the round's arithmetic each (20 rows, V
-// 128256: 29.3 us a call with the running max moved per group and 256 threads,
-// 17.2 with it moved per round, 13.0 with 512 threads), for many the memory
-// stream (4096 bf16 rows, V 163840: 246 -> 234 us, 5.7 TB/s).
+// ---- a row streamed once by NT threads ----
+// Per lane: the running max om, the first group bg that reached it, and os =
+// sum exp(v - om) (f32 group sums of exp2 accumulated in f64). The terms are
+// 2^fma(v, K, b) with b = RN(-om K): they share the exponent error e_b = om K +
+// b (exact, by an fma), which corr = 2^-e_b takes out (without it a logit of
+// magnitude 100 would cost ~5e-6 in log z).
+//
+// A row's time is its rounds of NT x U 16-byte groups: for few rows a memory
+// latency and the round's arithmetic each (20 rows, V 128256: 29.3 us a call
+// with the running max moved per group and 256 threads, 17.2 with it moved per
+// round, 13.0 with 512 threads), for many the memory stream (4096 bf16 rows, V
+// 163840: 246 -> 234 us, 5.7 TB/s).
+struct RowLane {
+    float om;
+    double os;
+    uint32_t bg;
+};
 template <int G, int NT>
-__global__ __launch_bounds__(NT) void verify_kernel(VerifyArgs a) {
+__device__ __forceinline__ RowLane stream_row(const void* rowp, uint32_t V) {
     constexpr int U = 8;                   // 16-byte groups in flight per thread
     constexpr float kL2E = 1.4426950408889634f;
-    __shared__ float redf[NT / kWave];
-    __shared__ uint32_t redu[NT / kWave];
-    __shared__ double redd[NT / kWave];
-    const uint32_t rows = a.n_seq * a.rows_per_seq;
-    const uint32_t row = wg_x();
-    if (row >= rows) return;
-    const uint32_t V = a.vocab;
-    const uint32_t esz = a.dtype == LCS_BF16 ? 2u : 4u;
-    const void* rowp = static_cast<const char*>(a.logits) + (uint64_t)row * a.row_stride * esz;
     const float NEG = -__builtin_huge_valf();
-
-    // per lane: running max om, the first group bg that reached it, and
-    // os = sum exp(v - om) (f32 group sums of exp2 accumulated in f64). The
-    // terms are 2^fma(v, K, b) with b = RN(-om K): they share the exponent
-    // error e_b = om K + b (exact, by an fma), which corr = 2^-e_b takes out
-    // (without it a logit of magnitude 100 would cost ~5e-6 in log z)
     const uint32_t ng = (V + G - 1) / G;
     float om = NEG, b = 0.0f;
     double os = 0.0, corr = 1.0;
@@ -94,20 +91,44 @@ __global__ __launch_bounds__(NT) void verify_kernel(VerifyArgs a) {
             }
         }
     }
+    return RowLane{om, os, bg};
+}
+
+// The block's max and its first index, and the row's sum of exponentials
+// against it (NT threads; red*: NT / kWave entries).
+template <int G, int NT>
+__device__ __forceinline__ double reduce_row(const RowLane& l, const void* rowp, uint32_t V, float& bm, uint32_t& idx,
+                                             float* redf, uint32_t* redu, double* redd) {
     // first index of the lane max inside its first group
-    uint32_t idx = 0xfffffffeu;
-    if (bg != 0xffffffffu) {
+    idx = 0xfffffffeu;
+    if (l.bg != 0xffffffffu) {
         float v[G];
-        decode<G>(load16(rowp, bg), v);
+        decode<G>(load16(rowp, l.bg), v);
         uint32_t k = G;
 #pragma unroll
-        for (int j = G - 1; j >= 0; --j) k = (bg * G + j < V && v[j] == om) ? (uint32_t)j : k;
-        idx = bg * G + k;
+        for (int j = G - 1; j >= 0; --j) k = (l.bg * G + j < V && v[j] == l.om) ? (uint32_t)j : k;
+        idx = l.bg * G + k;
     }
-    float bm = om;
+    bm = l.om;
     block_argmax<NT>(bm, idx, redf, redu);
-    const double sc = om == NEG ? 0.0 : os * exp((double)om - (double)bm);
-    const double z = block_sum<NT>(sc, redd);
+    const double sc = l.om == -__builtin_huge_valf() ? 0.0 : l.os * exp((double)l.om - (double)bm);
+    return block_sum<NT>(sc, redd);
+}
+
+template <int G, int NT>
+__global__ __launch_bounds__(NT) void verify_kernel(VerifyArgs a) {
+    __shared__ float redf[NT / kWave];
+    __shared__ uint32_t redu[NT / kWave];
+    __shared__ double redd[NT / kWave];
+    const uint32_t rows = a.n_seq * a.rows_per_seq;
+    const uint32_t row = wg_x();
+    if (row >= rows) return;
+    const uint32_t V = a.vocab;
+    const void* rowp = static_cast<const char*>(a.logits) + (uint64_t)row * a.row_stride * (16u / G);
+    const RowLane l = stream_row<G, NT>(rowp, V);
+    float bm;
+    uint32_t idx;
+    const double z = reduce_row<G, NT>(l, rowp, V, bm, idx, redf, redu, redd);
     if (tid_x() == 0) {
         const double log_z = log(z) + (double)bm;
         const int32_t d = a.draft[row];
@@ -116,6 +137,128 @@ __global__ __launch_bounds__(NT) void verify_kernel(VerifyArgs a) {
         a.draft_lp[row] = lp;
         a.argmax_ids[row] = (int32_t)(idx < V ? idx : 0u);
     }
+}
+
+// ---- logprobs_from over many rows (sampling.cpp:150-190) ----
+// A workgroup per row streams it once and writes its argmax, chosen's logprob
+// and the top n. The n-th largest of 64 sets of lanes' maxima bounds the row's
+// n-th largest value from below, so the candidates lie in the lanes whose max
+// reaches it (about n): their groups are read again, a group per lane of a wave,
+// and the candidates ranked. A row with more lanes or candidates than fit
+// (hundreds of values tied at the top) finds its top n one by one, each the
+// best rank key after the last. 1024 bf16
+// rows of V 128256, top 5: 99.8 us on the sliced path (85 + 18) -> 55.1, 4.8 TB/s.
+constexpr int kLpThreads = 512;
+constexpr uint32_t kLpLanes = 64, kLpCand = 256;   // lanes read again, candidates ranked
+template <int G>
+__global__ __launch_bounds__(kLpThreads) void logprobs_kernel(LogprobArgs a) {
+    constexpr int NT = kLpThreads, NW = NT / kWave;
+    __shared__ float redf[NW];
+    __shared__ uint32_t redu[NW];
+    __shared__ double redd[NW];
+    __shared__ uint64_t redk[NW];
+    __shared__ float lmax[NT];
+    __shared__ uint32_t nl, nc, lanes[kLpLanes];
+    __shared__ uint64_t ck[kLpCand];
+    __shared__ double log_z_s;
+    const uint32_t tid = tid_x(), row = wg_x();
+    const int lane = lane_id(), wv = __builtin_amdgcn_readfirstlane((int)(tid / kWave));
+    if (row >= a.rows) return;
+    const uint32_t V = a.vocab, ng = (V + G - 1) / G, ntop = a.n_top;
+    const void* rowp = static_cast<const char*>(a.logits) + (uint64_t)row * a.row_stride * (16u / G);
+    const RowLane l = stream_row<G, NT>(rowp, V);
+    lmax[tid] = l.om;
+    if (tid == 0) { nl = 0u; nc = 0u; }
+    float bm;
+    uint32_t idx;
+    const double z = reduce_row<G, NT>(l, rowp, V, bm, idx, redf, redu, redd);   // (its barriers order lmax, nl, nc)
+    if (tid == 0) {
+        const double log_z = log(z) + (double)bm;
+        log_z_s = log_z;
+        const uint32_t am = idx < V ? idx : 0u;
+        if (a.ids) a.ids[row] = (int32_t)am;
+        const int32_t d = a.chosen ? a.chosen[row] : (int32_t)am;
+        const bool in = d >= 0 && (uint32_t)d < V;
+        a.chosen_lp[row] = in ? (float)((double)load_elem(rowp, G == 8 ? LCS_BF16 : LCS_F32, (uint32_t)d) - log_z) : 0.0f;
+    }
+    if (ntop == 0u) return;   // (uniform)
+    float m = lmax[lane];
+#pragma unroll
+    for (int w = 1; w < NW; ++w) m = fmaxf(m, lmax[lane + w * kWave]);
+    // (every wave finds the same bound, the keys cut to 16 bits from below)
+    const uint32_t k1 = fkey(m) >> 16;
+    uint32_t T = 0;
+#pragma unroll
+    for (int sh = 14; sh >= 0; sh -= 2) {
+        const uint32_t T1 = T | (1u << sh), T2 = T | (2u << sh), T3 = T | (3u << sh);
+        const uint32_t c1 = (uint32_t)__builtin_popcountll(ballot(k1 >= T1));
+        const uint32_t c2 = (uint32_t)__builtin_popcountll(ballot(k1 >= T2));
+        const uint32_t c3 = (uint32_t)__builtin_popcountll(ballot(k1 >= T3));
+        T = c3 >= ntop ? T3 : c2 >= ntop ? T2 : c1 >= ntop ? T1 : T;
+    }
+    const float t = key_to_f(max(T << 16, 0x007fffffu));   // (>= -inf)
+    if (l.om >= t) {
+        const uint32_t s = atomicAdd(&nl, 1u);
+        if (s < kLpLanes) lanes[s] = tid;
+    }
+    __syncthreads();
+    const uint32_t n_lanes = nl;
+    if (n_lanes <= kLpLanes) {
+        for (uint32_t i = (uint32_t)wv; i < n_lanes; i += NW) {
+            for (uint32_t g = lanes[i] + (uint32_t)lane * NT; g < ng; g += kWave * NT) {
+                float v[G];
+                decode<G>(load16(rowp, g), v);
+#pragma unroll
+                for (int k = 0; k < G; ++k) {
+                    if (v[k] >= t && g * G + k < V) {
+                        const uint32_t s = atomicAdd(&nc, 1u);
+                        if (s < kLpCand) ck[s] = rank_key(v[k], g * G + k);
+                    }
+                }
+            }
+        }
+    }
+    __syncthreads();
+    const double log_z = log_z_s;
+    auto put = [&](uint32_t r, uint64_t key) {
+        a.top_ids[(uint64_t)row * ntop + r] = (int32_t)rank_idx(key);
+        a.top_lp[(uint64_t)row * ntop + r] = (float)((double)rank_val(key) - log_z);
+    };
+    const uint32_t have = min(ntop, V);   // (past the vocabulary: no key)
+    if (n_lanes <= kLpLanes && nc <= kLpCand) {   // (uniform)
+        if (wv == 0) {
+            uint64_t k[4];
+            uint32_t rk[4];
+            lds_rank4(ck, nc, k, rk);
+#pragma unroll
+            for (int c = 0; c < 4; ++c) {
+                if ((uint32_t)lane + (uint32_t)c * kWave < nc && rk[c] < ntop) put(rk[c], k[c]);
+            }
+        }
+    } else {
+        uint64_t last = 0ull;
+        for (uint32_t r = 0; r < have; ++r) {
+            uint64_t best = ~0ull;
+            for (uint32_t g = tid; g < ng; g += NT) {
+                float v[G];
+                decode<G>(load16(rowp, g), v);
+#pragma unroll
+                for (int k = 0; k < G; ++k) {
+                    const uint64_t key = rank_key(v[k], g * G + k);
+                    if (g * G + k < V && (r == 0u || key > last)) best = u64_min(best, key);
+                }
+            }
+            last = block_min_u64<NT>(best, redk);
+            if (tid == 0) put(r, last);
+        }
+    }
+    if (wv == 0 && (uint32_t)lane >= have && (uint32_t)lane < ntop) put((uint32_t)lane, ~0ull);
+}
+
+hipError_t launch_logprobs(const LogprobArgs& a, uint32_t dtype, hipStream_t st) {
+    if (dtype == LCS_BF16) hipLaunchKernelGGL(logprobs_kernel<8>, dim3(a.rows), dim3(kLpThreads), 0, st, a);
+    else hipLaunchKernelGGL(logprobs_kernel<4>, dim3(a.rows), dim3(kLpThreads), 0, st, a);
+    return hipGetLastError();
 }
 
 // Acceptance length per sequence (engine.cpp:366-383): leading rows whose
