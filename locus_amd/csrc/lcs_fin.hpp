@@ -632,6 +632,11 @@ __device__ __forceinline__ bool fin_decide(const SampleArgs& a, uint32_t row, Fi
     return false;
 }
 
+// What is left of a row after fin_row.
+constexpr uint32_t kFinDone = 0u;    // nothing, or another path's row
+constexpr uint32_t kFinExact = 1u;   // all of it
+constexpr uint32_t kFinRest = 2u;    // the decision (see fin_row's end)
+
 // The finalize of one row on the sliced path: the row's records merged and the
 // row resolved (see lcs_slice.hip's header), by a workgroup of kFinThreads
 // threads. Returns early for rows of other paths. row_fin calls it at kernel
@@ -639,7 +644,7 @@ __device__ __forceinline__ bool fin_decide(const SampleArgs& a, uint32_t row, Fi
 // parameters arrive (a row of another path reads a stale record, unused, and
 // returns).
 template <int G, bool TK>
-__device__ __forceinline__ void fin_row(const lcs_params* params, const uint64_t* srecs, uint32_t row, uint32_t vocab,
+__device__ __forceinline__ uint32_t fin_row(const lcs_params* params, const uint64_t* srecs, uint32_t row, uint32_t vocab,
                                         uint32_t flags, uint32_t slices, uint32_t n_top, const SampleArgs& a,
                                         FinSmem& sm) {
 #ifdef LCS_PROFILE
@@ -679,18 +684,15 @@ __device__ __forceinline__ void fin_row(const lcs_params* params, const uint64_t
     const lcs_params P = scalar_load(params + row);
     const bool masked = a.mask != nullptr && (a.has_mask == nullptr || scalar_load_u8(a.has_mask + row) != 0);
     const uint32_t mode = row_mode(P, masked, vocab);
-    if (mode != kModeGreedy && mode != kModeWindow && mode != kModeTopK) return;
+    if (mode != kModeGreedy && mode != kModeWindow && mode != kModeTopK) return kFinDone;
     // a slice that could not take all its penalised groups as exceptions, or
     // that left the row out, sends the row to the exact path (every wave
     // holds the same headers, so the test is uniform)
     if (ballot((uint32_t)lane < S && ((uint32_t)(hd[0] >> 48) & (rec::kFlagPenOverflow | rec::kFlagExact)) != 0u)) {
-        stage_args(&sm.args, a);
-        exact_row<kFinThreads, kFinFbBins, kFinFbCap, kFbHistCap, G>(sm.args, row, sm.u.ex);
-        return;
+        return kFinExact;
     }
     PROF_AT(kProfFin + row, 20 + wv);
     const bool stoch = mode == kModeWindow, topk = mode == kModeTopK;
-    if ((flags & kFlagNucAfter) != 0u && stoch && tid == 0) const_cast<uint64_t*>(srecs)[wide_flag_at(row)] = 0ull;
     const float inv_t = stoch || topk ? fdiv(1.0f, P.temperature) : 1.0f;
     const double u = (stoch || topk) && wv == 0 ? a.u[row] : 0.0;
     PROF_AT(kProfFin + row, 4 + wv);
@@ -747,7 +749,7 @@ __device__ __forceinline__ void fin_row(const lcs_params* params, const uint64_t
         };
         if (!(stoch || topk)) {
             if (tid == 0 && want_lp) write_lp();
-            return;
+            return kFinDone;
         }
         if (wv == 0) {
             fb = fin_decide(a, row, sm, topk ? LCS_PATH_TOPK : LCS_PATH_WINDOW, P, u);
@@ -759,35 +761,12 @@ __device__ __forceinline__ void fin_row(const lcs_params* params, const uint64_t
 #endif
         }
         __syncthreads();
-        if (!sm.fin_fb_decide) return;
+        if (!sm.fin_fb_decide) return kFinDone;
     }
-    // the records cannot settle this row. When the nucleus kernels follow,
-    // they take it with all its slices (64 rows of V 128256 whose windows hold
-    // thousands of ids: 117 us a call against 541 with exact_row's one workgroup a
-    // row); a penalty window above max_hist stays here, where it is reported
-    if ((flags & kFlagNucAfter) != 0u && stoch && !(want_lp && sm.fin_fb[1] != 0u)) {
-        const uint32_t hn = penalties_active(P) && a.hist_off != nullptr ? a.hist_off[row + 1] - a.hist_off[row] : 0u;
-        if (min(hn, P.repeat_last_n) <= a.max_hist) {   // (uniform)
-            if (tid == 0) const_cast<uint64_t*>(srecs)[wide_flag_at(row)] = 1ull;
-            return;
-        }
-    }
-    // else the exact single-workgroup path
-    // (out of line: it reads the kernel arguments from an LDS copy). Unless
-    // the log-normaliser's wave flagged the row, the records still give its
-    // penalised maximum and log-normaliser (and the top-n is written), and
-    // the exact path skips its stats pass (the top-n merge read the union
-    // that exact_row reuses: stage_args's barrier orders the two)
-    // (only window and top-k rows, unmasked, get here; the fields come from
-    // LDS so that nothing stays live across the finalize for them)
-    ExactPre pre{};
-    if (!(want_lp && sm.fin_fb[1] != 0u)) {
-        pre.on = 1u;
-        pre.maxl = sm.fin_premax;
-        pre.log_z = want_lp ? sm.log_z : 0.0;
-    }
-    stage_args(&sm.args, a);
-    exact_row<kFinThreads, kFinFbBins, kFinFbCap, kFbHistCap, G>(sm.args, row, sm.u.ex, pre);
+    // the records cannot settle the row; unless the log-normaliser's wave
+    // flagged it, they still give its penalised maximum and log-normaliser
+    // (and its top-n is written)
+    return !(want_lp && sm.fin_fb[1] != 0u) ? kFinRest : kFinExact;
 }
 
 // One workgroup per row (the sliced path's second kernel). The leading
@@ -813,7 +792,35 @@ __global__ __launch_bounds__(kFinThreads) void row_fin(const lcs_params* params,
         const WinStage st = scalar_load(a.wstage + row);
         if (st.flag == 1u) a.wh[st.slot] = st.hdr;
     }
-    fin_row<G, TK>(params, srecs, row, vocab, flags, slices, n_top, a, sm);
+    const uint32_t rest = fin_row<G, TK>(params, srecs, row, vocab, flags, slices, n_top, a, sm);
+    if (rest == kFinDone) return;   // (uniform)
+    // When the nucleus kernels follow, they take a window row with all its
+    // slices (64 rows of V 128256 whose windows hold thousands of ids: 117 us
+    // a call against 541 with exact_row's one workgroup a row); a penalty
+    // window above max_hist stays here, where it is reported
+    if ((flags & kFlagNucAfter) != 0u && rest == kFinRest) {
+        const lcs_params P = scalar_load(params + row);
+        const uint32_t hn = penalties_active(P) && a.hist_off != nullptr ? a.hist_off[row + 1] - a.hist_off[row] : 0u;
+        if (row_mode(P, false, vocab) == kModeWindow && min(hn, P.repeat_last_n) <= a.max_hist) {   // (uniform)
+            if (tid_x() == 0)
+                atomicOr(reinterpret_cast<uint32_t*>(a.srecs + (uint64_t)row * kRecsPerRow * rec::kWords64) + 1,
+                         rec::kFlagHanded << 16);
+            return;
+        }
+    }
+    // else the exact single-workgroup path (out of line: it reads the kernel
+    // arguments from an LDS copy), without its stats pass where the records
+    // give what that finds (the top-n merge read the union that exact_row
+    // reuses: stage_args's barrier orders the two; the fields come from LDS so
+    // that nothing stays live across the finalize for them)
+    ExactPre pre{};
+    if (rest == kFinRest) {
+        pre.on = 1u;
+        pre.maxl = sm.fin_premax;
+        pre.log_z = (flags & LCS_WANT_LOGPROBS) != 0 ? sm.log_z : 0.0;
+    }
+    stage_args(&sm.args, a);
+    exact_row<kFinThreads, kFinFbBins, kFinFbCap, kFbHistCap, G>(sm.args, row, sm.u.ex, pre);
 }
 
 }  // namespace lcs

@@ -51,17 +51,14 @@ constexpr uint32_t kFlagCandOverflow = 2u;         // more top-n candidates than
 constexpr uint32_t kFlagWinLost = 4u;              // more window entries than the slice could rank
 constexpr uint32_t kFlagPenOverflow = 8u;          // more penalised groups than the slice could take
 constexpr uint32_t kFlagExact = 16u;               // the row is resolved on the exact path
+constexpr uint32_t kFlagHanded = 32u;              // (first record) the nucleus kernels take the row
 }  // namespace rec
 
 // SampleArgs::flags: the nucleus kernels follow the sliced ones in this call and
-// take the window rows that their records cannot settle (row_fin sets the word
-// of such a row's first record at wide_flag_at). A flag bit, since the kernels
-// have the flags in registers from the start.
+// take the window rows that their records cannot settle (row_fin marks such a
+// row's first record with kFlagHanded, slice_stats writes that word anew in
+// every call). A flag bit, since the kernels have the flags in registers.
 constexpr uint32_t kFlagNucAfter = 1u << 31;
-__host__ __device__ inline uint64_t wide_flag_at(uint32_t row) {
-    static_assert(rec::kWinRaw + kWinCap < rec::kWords64, "a spare word");
-    return ((uint64_t)row * kRecsPerRow + 1u) * rec::kWords64 - 1u;
-}
 
 // ---- single-workgroup exact path ----
 constexpr int kGenThreads = 1024;

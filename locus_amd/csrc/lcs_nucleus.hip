@@ -387,7 +387,8 @@ __device__ __forceinline__ void nuc_taylor(float sx, double scale, bool minus_on
 __device__ __forceinline__ bool nuc_takes(const SampleArgs& a, uint32_t row, const lcs_params& P, bool masked) {
     const uint32_t mode = row_mode(P, masked, a.vocab);
     if (mode == kModeNucleus) return true;
-    return mode == kModeWindow && (a.flags & kFlagNucAfter) != 0u && scalar_load(a.srecs + wide_flag_at(row)) != 0ull;
+    return mode == kModeWindow && (a.flags & kFlagNucAfter) != 0u &&
+           ((scalar_load(a.srecs + (uint64_t)row * kRecsPerRow * rec::kWords64) >> 48) & rec::kFlagHanded) != 0ull;
 }
 
 // Row and mode of a finalize workgroup (one per row of the launch); false
