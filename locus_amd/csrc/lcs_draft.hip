@@ -7,14 +7,16 @@
 // it is empty when ngram or max_draft is 0, when the context is not longer
 // than ngram, or when the trailing n-gram does not occur earlier.
 //
-// The workgroup stages the trailing n-gram in LDS and tests candidate starts
-// from the most recent backwards, kDraftChunk starts per round: the round's
+// The workgroup (NT threads) stages the trailing n-gram in LDS and tests
+// candidate starts from the most recent backwards, 16 NT starts per round: the round's
 // tokens (its starts and the ngram - 1 tokens after the last one) are loaded
 // into LDS at once, coalesced, all loads issued before the first is used; each
-// thread then tests 16 starts (s = lo + t + 256 j) from LDS, one pattern
+// thread then tests 16 starts (s = lo + t + NT j) from LDS, one pattern
 // token at a time, until no lane of its wave has a start left. The round's
 // largest matching start is the answer when there is one; otherwise the next
-// round takes the kDraftChunk starts before it.
+// round takes the 16 NT starts before it. A round is a memory round trip and
+// about as much arithmetic, so a long context goes by its rounds (see
+// launch_draft).
 #include <hip/hip_runtime.h>
 #include <stdint.h>
 
@@ -23,13 +25,13 @@
 
 namespace lcs {
 
-constexpr int kDraftThreads = 256;
 constexpr uint32_t kDraftPer = 16;                          // starts per thread per round
-constexpr uint32_t kDraftChunk = kDraftThreads * kDraftPer;  // starts per round
-constexpr uint32_t kDraftTok = kDraftChunk + kDraftMaxNgram; // tokens a round stages (rounded up below)
-constexpr uint32_t kDraftLoads = (kDraftTok + kDraftThreads - 1) / kDraftThreads;
 
+template <int kDraftThreads>
 __global__ __launch_bounds__(kDraftThreads) void ngram_draft_kernel(DraftArgs a) {
+    constexpr uint32_t kDraftChunk = kDraftThreads * kDraftPer;   // starts per round
+    constexpr uint32_t kDraftTok = kDraftChunk + kDraftMaxNgram;  // tokens a round stages (rounded up below)
+    constexpr uint32_t kDraftLoads = (kDraftTok + kDraftThreads - 1) / kDraftThreads;
     __shared__ int32_t pat[kDraftMaxNgram];
     __shared__ int32_t tok[kDraftLoads * kDraftThreads];
     __shared__ uint32_t red[kDraftThreads / kWave];
@@ -61,7 +63,7 @@ __global__ __launch_bounds__(kDraftThreads) void ngram_draft_kernel(DraftArgs a)
 #pragma unroll
             for (uint32_t i = 0; i < kDraftLoads; ++i) tok[tid + i * (uint32_t)kDraftThreads] = v[i];
             __syncthreads();
-            // bit j: start lo + tid + 256 j is in the round and still matches
+            // bit j: start lo + tid + NT j is in the round and still matches
             uint32_t mm = 0;
 #pragma unroll
             for (uint32_t j = 0; j < kDraftPer; ++j) mm |= (lo + tid + j * (uint32_t)kDraftThreads < hi) ? 1u << j : 0u;
@@ -70,7 +72,7 @@ __global__ __launch_bounds__(kDraftThreads) void ngram_draft_kernel(DraftArgs a)
                 uint32_t keep = 0;
 #pragma unroll
                 for (uint32_t j = 0; j < kDraftPer; ++j) {
-                    // (in bounds for every j: tid + 256 j + k < kDraftChunk + kDraftMaxNgram)
+                    // (in bounds for every j: tid + NT j + k < kDraftChunk + kDraftMaxNgram)
                     keep |= tok[tid + j * (uint32_t)kDraftThreads + k] == pk ? 1u << j : 0u;
                 }
                 mm &= keep;
@@ -100,8 +102,17 @@ __global__ __launch_bounds__(kDraftThreads) void ngram_draft_kernel(DraftArgs a)
     if (tid == 0) a.draft_len[seq] = len;
 }
 
+// Threads per sequence: the contexts' lengths are known on the device only, so
+// the number of sequences decides: a CU each, 1024 threads; above, 512, two a
+// CU (us a call with 256 / 512 / 1024 threads, contexts up to 32768 tokens: 64
+// sequences 12.1 / 8.2 / 7.2, 256: 14.2 / 9.1 / 7.5, 512: 17.2 / 12.6 / 13.7; up
+// to 131072 tokens, one sequence 11.3 / 8.1 / 7.5, 512: 57 / 39 / 33; 512 of up
+// to 4096: 6.0 / 6.1 / 7.9). Above 1024 sequences the small workgroups share
+// the CUs as they are.
 hipError_t launch_draft(const DraftArgs& a, hipStream_t st) {
-    hipLaunchKernelGGL(ngram_draft_kernel, dim3(a.n_seq), dim3(kDraftThreads), 0, st, a);
+    if (a.n_seq <= 256u) hipLaunchKernelGGL(ngram_draft_kernel<1024>, dim3(a.n_seq), dim3(1024), 0, st, a);
+    else if (a.n_seq <= 1024u) hipLaunchKernelGGL(ngram_draft_kernel<512>, dim3(a.n_seq), dim3(512), 0, st, a);
+    else hipLaunchKernelGGL(ngram_draft_kernel<256>, dim3(a.n_seq), dim3(256), 0, st, a);
     return hipGetLastError();
 }
 

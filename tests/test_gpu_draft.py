@@ -100,3 +100,24 @@ def test_draft_rejects_bad_arguments(sampler):
         sampler.ngram_draft([[1, 2, 3]], 65, 4)
     with pytest.raises(SamplerError):
         sampler.ngram_draft([[1, 2, 3]], 2, 257)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("n_seq,chunk", [(3, 16384), (256, 16384), (257, 8192), (1025, 4096)])
+def test_draft_workgroup_sizes(sampler, n_seq, chunk):
+    """Each workgroup size at the edges of its rounds (16 starts a thread): the
+    only match one start before, at and after a round's border, the first
+    start of all, and none."""
+    ng, md = 3, 5
+    ctxs = []
+    for i in range(n_seq):
+        n = (chunk, chunk + ng, chunk + ng + 1, 2 * chunk + ng, 17)[i % 5] if i < 10 else 20 + i % 9
+        c = np.arange(1000, 1000 + n, dtype=np.int32)   # no n-gram recurs
+        starts = n - ng
+        at = (starts - chunk - 1, starts - chunk, starts - chunk + 1, 0, None)[(i // 5 + i) % 5] if i < 10 else (i % 4 or None)
+        if at is not None and 0 <= at < starts - ng:
+            c[at:at + ng] = c[n - ng:]
+        ctxs.append(c.tolist())
+    got, _ = sampler.ngram_draft(ctxs, ng, md)
+    for c, g in zip(ctxs, got):
+        assert g == O.ngram_draft(c, ng, md), len(c)
