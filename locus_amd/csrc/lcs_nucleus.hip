@@ -74,19 +74,15 @@ struct NucLocal {
     float mpen[kNW], npen[kNW], mmsk[kNW], nmsk[kNW], nraw[kNW];
     uint32_t ipen[kNW], imsk[kNW], nall[kNW];
     uint64_t ck[kNucCand];
-    // select-pass finalize
-    uint32_t ngc[2];           // group sizes of alternate gathers (each reset one gather ahead)
-    uint32_t fp_pos;           // first_prefix's position and prefix mass
-    double fp_m;
-    uint32_t lg_n, lg_cb;      // nuc_large_group: candidates left, and the count and weight before them
-    double lg_mb;
-    uint32_t out_flag;
     // the row state pass B's workgroups derive from pass A's records
     float st_maxl, st_sx;
     uint32_t st_use_mask, st_fallback, st_off;
-    NucRange rgl[kNucRanges];  // the planned ranges, for lookups by a computed index (select finalize)
-    SampleArgs args;           // for the exact fallback
 };
+// The select finalize's block: kFT threads, one workgroup a row, so that its
+// chain of passes over the row's list is short (512 against 256 threads: 256 top-p
+// rows 17.4 -> 12.9 us, 64 wide min-p rows 22.1 -> 17.6, 24 mixed rows 24.4 -> 19.9).
+constexpr int kFT = 512;
+constexpr int kFW = kFT / kWave;
 struct NucFinC {
     uint32_t scnt[kNucRanges][kNucSub];   // sub-bin counts, then inclusive
     double smass[kNucRanges][kNucSub];    // sub-bin masses, then inclusive
@@ -106,13 +102,31 @@ struct NucSmem {
             uint64_t top[kMaxSlices * kTopMax];   // top-n merge (pass B finalize, wave 1)
         } h;                              // histogram (pass B finalize)
         uint64_t pk[kNucBins];            // histogram (pass B): packed count and mass per bin
-        NucFinC fc;                       // select finalize
-        ExactSmem<kSliceThreads, kFbBins, kFbCap, kFbHistCap> ex;
     } u;
     NucLocal l;
 };
 __shared__ NucSmem g_nuc;
-static_assert(sizeof(NucFinC) <= sizeof(uint32_t) * kSliceMax, "the select finalize's LDS fits the union");
+
+struct NucFinSmem {
+    union {
+        NucFinC fc;
+        ExactSmem<kFT, kFbBins, kFbCap, kFbHistCap> ex;
+    } u;
+    struct {
+        uint32_t ngc[2];           // group sizes of alternate gathers (each reset one gather ahead)
+        uint32_t fp_pos;           // first_prefix's position and prefix mass
+        double fp_m;
+        uint32_t lg_n, lg_cb;      // nuc_large_group: candidates left, and the count and weight before them
+        double lg_mb;
+        uint32_t out_flag;
+        uint32_t nall[kFW], ipen[kFW], imsk[kFW];   // per wave: counts, buckets
+        double sraw[kFW];                           // and masses
+        uint64_t ck[kFW];                           // and keys
+        NucRange rgl[kNucRanges];  // the planned ranges, for lookups by a computed index
+        SampleArgs args;           // for the exact fallback
+    } l;
+};
+__shared__ NucFinSmem g_fin;   // (the select finalize alone references it)
 
 // The select finalize's code of each compacted candidate: range k and
 // sub-bin s as k * kNucSub + s, kNoCode outside the planned ranges. Only
@@ -818,9 +832,7 @@ __global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(4))) void nu
     const uint32_t cm = in.cand_bits(use_mask);
     const bool all_cand = ballot(cm != 0xffffffffu) == 0u;
     const double two_k = 68719476736.0 * (double)sx;   // 2^36 sx
-    double off_m = 0.0;
-    uint32_t off_n = 0u;
-    auto fill = [&](auto deg, auto all, auto past) {
+    auto fill = [&](auto deg, auto all, auto past, double& off_m, uint32_t& off_n) {
         constexpr int n = decltype(deg)::value;
         constexpr bool off_grid = n == 8;   // (only when sx = 4: f may pass kNucBins)
         double q[n + 1];   // (exp(d) - 1) 2^k
@@ -851,10 +863,12 @@ __global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(4))) void nu
     using D8 = std::integral_constant<int, 8>;
     using Yes = std::true_type;
     using No = std::false_type;
-    if (sm.l.st_off) {
-        if (sx >= 64.0f) fill(D5{}, No{}, Yes{});
-        else if (sx >= 16.0f) fill(D6{}, No{}, Yes{});
-        else fill(D8{}, No{}, Yes{});
+    auto past_bins = [&]() {
+        double off_m = 0.0;
+        uint32_t off_n = 0u;
+        if (sx >= 64.0f) fill(D5{}, No{}, Yes{}, off_m, off_n);
+        else if (sx >= 16.0f) fill(D6{}, No{}, Yes{}, off_m, off_n);
+        else fill(D8{}, No{}, Yes{}, off_m, off_n);
         off_m = block_sum<NT>(off_m, sm.l.sraw);
         off_n = block_sum_u<NT>(off_n, sm.l.nall);
         if (tid == 0) {
@@ -862,15 +876,20 @@ __global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(4))) void nu
             orec[0] = d_bits(off_m);
             orec[1] = off_n;
         }
+    };
+    double unused_m = 0.0;
+    uint32_t unused_n = 0u;
+    if (__builtin_expect(sm.l.st_off != 0u, 0)) {
+        past_bins();
     } else if (sx >= 64.0f) {
-        if (all_cand) fill(D5{}, Yes{}, No{});
-        else fill(D5{}, No{}, No{});
+        if (all_cand) fill(D5{}, Yes{}, No{}, unused_m, unused_n);
+        else fill(D5{}, No{}, No{}, unused_m, unused_n);
     } else if (sx >= 16.0f) {
-        if (all_cand) fill(D6{}, Yes{}, No{});
-        else fill(D6{}, No{}, No{});
+        if (all_cand) fill(D6{}, Yes{}, No{}, unused_m, unused_n);
+        else fill(D6{}, No{}, No{}, unused_m, unused_n);
     } else {
-        if (all_cand) fill(D8{}, Yes{}, No{});
-        else fill(D8{}, No{}, No{});
+        if (all_cand) fill(D8{}, Yes{}, No{}, unused_m, unused_n);
+        else fill(D8{}, No{}, No{}, unused_m, unused_n);
     }
     __syncthreads();
     uint64_t* gp = a.nh_pk + ((uint64_t)wrow * kMaxSlices + slice) * kNucBins;
@@ -937,12 +956,16 @@ __global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(1, 2))) void
         // out of its count for the mass, their own mass in
         double off_m = 0.0;
         uint32_t off_n = 0u;
-        if ((nr->flags & kNucOff) && tid == NT - 1) {
-            const uint64_t* orec = reinterpret_cast<const uint64_t*>(a.recs) + (uint64_t)row * S * rec::kWords64 + nrec::kOff;
-            for (uint32_t ss = 0; ss < S; ++ss) {
-                off_m += bits_d(orec[(uint64_t)ss * rec::kWords64]);
-                off_n += (uint32_t)orec[(uint64_t)ss * rec::kWords64 + 1];
-            }
+        if ((nr->flags & kNucOff) && tid >= NT - kWave) {   // (the last wave, slice ss in lane ss)
+            static_assert(kMaxSlices <= kWave, "a slice per lane");
+            const uint32_t ss = tid - (NT - kWave);
+            const uint64_t* orec = reinterpret_cast<const uint64_t*>(a.recs) +
+                                   ((uint64_t)row * S + (ss < S ? ss : 0u)) * rec::kWords64 + nrec::kOff;
+            const double om = bits_d(orec[0]);
+            const uint32_t on = (uint32_t)orec[1];
+            off_m = wave_sum(ss < S ? om : 0.0);
+            off_n = wave_sum_u(ss < S ? on : 0u);
+            if (tid != NT - 1) { off_m = 0.0; off_n = 0u; }
         }
 #pragma unroll
         for (uint32_t k = 0; k < BPT; ++k) {
@@ -1109,7 +1132,7 @@ struct NucTarget {
     uint32_t pos;
     double before, norm, reach;
 };
-// A decisive group larger than kGroupMax (the candidates with codes c0..c1):
+// A decisive group larger than kGroupMax (the ng candidates with codes c0..c1):
 // narrowed to the at most kGroupMax candidates around its target, which are
 // ranked into gsorted with their weights in gw as the select finalize's gather
 // leaves a small group. Returns how many, with the group's candidates and
@@ -1125,39 +1148,64 @@ struct NucTarget {
 // nuc_select_fin_kernel 1090 -> 26 us, the call 1122 -> 73 us. Out of line:
 // inlined at the three decisions it cost a call without a large group (32
 // masked rows) 0.6 of 42.7 us.
-__device__ __attribute__((noinline)) uint32_t nuc_large_group(uint32_t c0, uint32_t c1, uint32_t n,
+__device__ __attribute__((noinline)) uint32_t nuc_large_group(uint32_t c0, uint32_t c1, uint32_t ng, uint32_t n,
                                                               const uint64_t* list, float maxl, float inv_t,
                                                               NucTarget tgt) {
-    NucSmem& sm = g_nuc;
+    NucFinSmem& sm = g_fin;
     const uint32_t tid = tid_x();
     const int lane = lane_id(), wv = (int)(tid / kWave);
     uint32_t* bc = reinterpret_cast<uint32_t*>(sm.u.fc.gsorted);   // (both free: the group is not ranked yet)
     double* bm = sm.u.fc.gw;
-    static_assert(kGroupMax == NT && kNW == 4, "one bucket and one group candidate per thread");
+    static_assert(kGroupMax == 4 * kWave && kGroupMax <= kFT, "a bucket per thread of the first four waves");
+    constexpr int kBW = (int)kGroupMax / kWave;
+    const bool bucket = tid < kGroupMax;
     uint64_t glo = 0ull, ghi = ~0ull;   // the keys left
     uint32_t cb = 0u, m = kNone;
     double mb = 0.0;
-    auto each = [&](auto body) {
-        for (uint32_t i = tid; i < n; i += NT) {
+    auto from_list = [&](auto body) {
+        for (uint32_t i = tid; i < n; i += kFT) {
             const uint32_t c = g_code[i];
-            if (c >= c0 && c <= c1) {
-                const uint64_t key = i < kNucKeyCache ? g_nuc.u.fc.lkey[i] : list[i];
+            if (c >= c0 && c <= c1) body(i < kNucKeyCache ? g_fin.u.fc.lkey[i] : list[i]);
+        }
+    };
+    // the group's keys copied to the unused half of the codes, when both fit:
+    // the steps then go over the group instead of the row's list (24 mixed
+    // bf16 rows: this kernel 26.3 -> 24.4 us)
+    uint64_t* buf = reinterpret_cast<uint64_t*>(&g_code[kNucList / 2]);
+    constexpr uint32_t kBuf = kNucList / 2 * sizeof(uint16_t) / sizeof(uint64_t);
+    const bool held = n <= kNucList / 2 && ng <= kBuf;   // (uniform)
+    if (held) {
+        if (tid == 0) sm.l.lg_n = 0u;
+        __syncthreads();
+        from_list([&](uint64_t key) { buf[atomicAdd(&g_fin.l.lg_n, 1u)] = key; });
+        __syncthreads();
+    }
+    auto each = [&](auto body) {
+        if (held) {
+            for (uint32_t i = tid; i < ng; i += kFT) {
+                const uint64_t key = buf[i];
                 if (key >= glo && key <= ghi) body(key);
             }
+        } else {
+            from_list([&](uint64_t key) {
+                if (key >= glo && key <= ghi) body(key);
+            });
         }
     };
     // (each step cuts the keys' range by 2^7 or more, unless the target meets
     // the gap between two clusters of keys within the sums' rounding)
     for (int it = 0; it < 10 && m > kGroupMax; ++it) {
-        bc[tid] = 0u;
-        bm[tid] = 0.0;
+        if (bucket) {
+            bc[tid] = 0u;
+            bm[tid] = 0.0;
+        }
         uint64_t kmin = ~0ull, nmax = ~0ull;
         each([&](uint64_t key) {
             kmin = u64_min(kmin, key);
             nmax = u64_min(nmax, ~key);
         });
-        kmin = block_min_u64<NT>(kmin, sm.l.ck);
-        const uint64_t kmax = ~block_min_u64<NT>(nmax, sm.l.ck);
+        kmin = block_min_u64<kFT>(kmin, sm.l.ck);
+        const uint64_t kmax = ~block_min_u64<kFT>(nmax, sm.l.ck);
         const int bits = 64 - __builtin_clzll((kmax - kmin) | 1ull);
         const int sh = bits > 8 ? bits - 8 : 0;
         each([&](uint64_t key) {
@@ -1167,22 +1215,22 @@ __device__ __attribute__((noinline)) uint32_t nuc_large_group(uint32_t c0, uint3
         });
         __syncthreads();
         // inclusive prefix sums over the buckets (bucket tid)
-        const uint32_t cl = bc[tid];
-        const double ml = bm[tid];
+        const uint32_t cl = bucket ? bc[tid] : 0u;
+        const double ml = bucket ? bm[tid] : 0.0;
         uint32_t ci = wave_scan_incl_u(cl);
         double mi = wave_scan_incl(ml);
         if (lane == kWave - 1) { sm.l.nall[wv] = ci; sm.l.sraw[wv] = mi; }
         __syncthreads();
         double mt = 0.0;
 #pragma unroll
-        for (int w = 0; w < kNW; ++w) {
+        for (int w = 0; w < kBW; ++w) {
             if (w < wv) { ci += sm.l.nall[w]; mi += sm.l.sraw[w]; }
             mt += sm.l.sraw[w];
         }
         // (the sums' rounding: at most n 2^-53 of the weight left, n <= kNucList)
         const double ge = 0x1p-37 * mt;
         auto met = [&](double p) { return (cb + ci - 1u >= tgt.pos) || (tgt.before + p) / tgt.norm >= tgt.reach; };
-        const uint64_t h0 = ballot(met(mb + mi + ge)), h1 = ballot(met(mb + mi - ge));
+        const uint64_t h0 = ballot(bucket && met(mb + mi + ge)), h1 = ballot(bucket && met(mb + mi - ge));
         if (lane == 0) {
             sm.l.ipen[wv] = h0 ? (uint32_t)wv * kWave + (uint32_t)__builtin_ctzll(h0) : kNone;
             sm.l.imsk[wv] = h1 ? (uint32_t)wv * kWave + (uint32_t)__builtin_ctzll(h1) : kNone;
@@ -1191,7 +1239,7 @@ __device__ __attribute__((noinline)) uint32_t nuc_large_group(uint32_t c0, uint3
         const uint32_t lastb = (uint32_t)((kmax - kmin) >> sh);
         uint32_t b0 = lastb, b1 = lastb;
 #pragma unroll
-        for (int w = 0; w < kNW; ++w) { b0 = min(b0, sm.l.ipen[w]); b1 = min(b1, sm.l.imsk[w]); }
+        for (int w = 0; w < kBW; ++w) { b0 = min(b0, sm.l.ipen[w]); b1 = min(b1, sm.l.imsk[w]); }
         if (tid == b0) { sm.l.lg_cb = cb + ci - cl; sm.l.lg_mb = mb + mi - ml; }
         if (tid == b1) sm.l.lg_n = cb + ci;
         __syncthreads();
@@ -1204,7 +1252,7 @@ __device__ __attribute__((noinline)) uint32_t nuc_large_group(uint32_t c0, uint3
     if (m > kGroupMax) return kNone;
     if (tid == 0) sm.l.lg_n = 0u;
     __syncthreads();   // (the buckets are read, lg_n is cleared)
-    each([&](uint64_t key) { g_nuc.u.fc.gkey[atomicAdd(&g_nuc.l.lg_n, 1u)] = key; });
+    each([&](uint64_t key) { g_fin.u.fc.gkey[atomicAdd(&g_fin.l.lg_n, 1u)] = key; });
     __syncthreads();
     if (tid < m) {
         const uint64_t x = sm.u.fc.gkey[tid];
@@ -1222,7 +1270,7 @@ __device__ __attribute__((noinline)) uint32_t nuc_large_group(uint32_t c0, uint3
 // row has to take the exact path.
 template <int G>
 __device__ __forceinline__ bool nuc_select_fin(const SampleArgs& a, uint32_t row) {
-    NucSmem& sm = g_nuc;
+    NucFinSmem& sm = g_fin;
     const uint32_t tid = tid_x();
     const int lane = lane_id(), wv = (int)(tid / kWave);
     const lcs_params P = scalar_load(a.params + row);
@@ -1247,13 +1295,13 @@ __device__ __forceinline__ bool nuc_select_fin(const SampleArgs& a, uint32_t row
     const uint32_t ncand = nr->n_cand;
     NPROF(row, 8);
     // sub-bin tables, bin scales
-    for (uint32_t i = tid; i < kNucRanges * kNucSub; i += NT) {
+    for (uint32_t i = tid; i < kNucRanges * kNucSub; i += kFT) {
         sm.u.fc.scnt[i / kNucSub][i % kNucSub] = 0u;
         sm.u.fc.smass[i / kNucSub][i % kNucSub] = 0.0;
     }
     {
         const double inv_sx = 1.0 / (double)sx;
-        for (uint32_t b = tid; b < kNucBins; b += NT) sm.u.fc.bscale[b] = exp_f64(-((double)b + 0.5) * inv_sx);
+        for (uint32_t b = tid; b < kNucBins; b += kFT) sm.u.fc.bscale[b] = exp_f64(-((double)b + 0.5) * inv_sx);
     }
     if (tid == 0) {
         sm.l.out_flag = n_all > kNucList ? 1u : 0u;
@@ -1290,17 +1338,17 @@ __device__ __forceinline__ bool nuc_select_fin(const SampleArgs& a, uint32_t row
     {
         // the first kNucKeyCache keys into LDS, every load issued before the
         // first is used (indices past n read entry 0 of the row's list, unused)
-        static_assert(kNucKeyCache % NT == 0, "key cache per thread");
-        constexpr uint32_t KP = kNucKeyCache / NT;
+        static_assert(kNucKeyCache % kFT == 0, "key cache per thread");
+        constexpr uint32_t KP = kNucKeyCache / kFT;
         uint64_t kq[KP];
 #pragma unroll
         for (uint32_t j = 0; j < KP; ++j) {
-            const uint32_t i = tid + j * NT;
+            const uint32_t i = tid + j * kFT;
             kq[j] = list[i < n ? i : 0u];
         }
 #pragma unroll
         for (uint32_t j = 0; j < KP; ++j) {
-            const uint32_t i = tid + j * NT;
+            const uint32_t i = tid + j * kFT;
             if (i < n) sm.u.fc.lkey[i] = kq[j];
         }
     }
@@ -1314,16 +1362,16 @@ __device__ __forceinline__ bool nuc_select_fin(const SampleArgs& a, uint32_t row
     // keys past the LDS cache come from the list in batches of PB per
     // thread, every load of a batch issued before the first is used
     constexpr uint32_t PB = 8;
-    for (uint32_t i0 = tid; i0 < n; i0 += PB * NT) {
+    for (uint32_t i0 = tid; i0 < n; i0 += PB * kFT) {
         uint64_t kb[PB];
 #pragma unroll
         for (uint32_t j = 0; j < PB; ++j) {
-            const uint32_t i = i0 + j * NT;
+            const uint32_t i = i0 + j * kFT;
             kb[j] = i < kNucKeyCache ? sm.u.fc.lkey[i] : list[i < n ? i : 0u];
         }
 #pragma unroll
         for (uint32_t j = 0; j < PB; ++j) {
-            const uint32_t i = i0 + j * NT;
+            const uint32_t i = i0 + j * kFT;
             if (i < n) {
                 uint32_t k, s, b;
                 float r;
@@ -1342,8 +1390,8 @@ __device__ __forceinline__ bool nuc_select_fin(const SampleArgs& a, uint32_t row
     __syncthreads();
     NPROF(row, 9);
     // inclusive sub-bin prefix sums, one wave per range (kNucSub = 2 per lane)
-    static_assert(kNucRanges == kNW && kNucSub == 2 * kWave, "one wave per range");
-    {
+    static_assert(kNucRanges <= kFW && kNucSub == 2 * kWave, "one wave per range");
+    if (wv < (int)kNucRanges) {
         const uint32_t k = (uint32_t)wv;
         const uint32_t c0 = sm.u.fc.scnt[k][2 * lane], c1 = sm.u.fc.scnt[k][2 * lane + 1];
         const double m0 = sm.u.fc.smass[k][2 * lane], m1 = sm.u.fc.smass[k][2 * lane + 1];
@@ -1393,7 +1441,7 @@ __device__ __forceinline__ bool nuc_select_fin(const SampleArgs& a, uint32_t row
         return false;
     };
     // Gathers the candidates of range k's sub-bins [s0, s1] into gkey and ranks
-    // them into gsorted with weights gw: P = 1, 2 or 4 adjacent threads rank
+    // them into gsorted with weights gw: P = 2 or 4 adjacent threads rank
     // one candidate, each against the keys j = p (mod P), joined by a quad
     // DPP sum. Every thread calls it.
     // (gather i counts into ngc[i & 1], which was cleared during gather i - 1,
@@ -1408,7 +1456,7 @@ __device__ __forceinline__ bool nuc_select_fin(const SampleArgs& a, uint32_t row
         // skipped, kNucList is a multiple of 4)
         const uint32_t c0 = k * kNucSub + s0, c1 = k * kNucSub + s1;
         static_assert(kNucList % 4 == 0, "code quads");
-        for (uint32_t i4 = 4 * tid; i4 < n; i4 += 4 * NT) {
+        for (uint32_t i4 = 4 * tid; i4 < n; i4 += 4 * kFT) {
             const uint2 cq = *reinterpret_cast<const uint2*>(&g_code[i4]);
 #pragma unroll
             for (uint32_t q = 0; q < 4; ++q) {
@@ -1421,9 +1469,9 @@ __device__ __forceinline__ bool nuc_select_fin(const SampleArgs& a, uint32_t row
         }
         __syncthreads();
         const uint32_t ng = *cnt;
-        static_assert(kGroupMax == NT, "one thread per group candidate at most");
+        static_assert(kGroupMax * 2 <= kFT, "two threads per group candidate or more");
         if (ng <= kGroupMax) {   // uniform
-            const uint32_t lp = ng <= kWave ? 2u : ng <= 2 * kWave ? 1u : 0u;   // P = 2^lp
+            const uint32_t lp = 4u * ng <= kFT ? 2u : 1u;   // P = 2^lp
             const uint32_t last = ng > 0u ? ng - 1u : 0u;
             const uint32_t kc = tid >> lp, p = tid & ((1u << lp) - 1u);
             const uint64_t x = sm.u.fc.gkey[min(kc, last)];
@@ -1440,7 +1488,7 @@ __device__ __forceinline__ bool nuc_select_fin(const SampleArgs& a, uint32_t row
 #pragma unroll
                 for (int u = 0; u < 8; ++u) rank += e[u] < x ? 1u : 0u;
             }
-            if (lp >= 1) rank += (uint32_t)dpp_i<0xB1>(0, (int)rank);   // quad_perm [1,0,3,2]
+            rank += (uint32_t)dpp_i<0xB1>(0, (int)rank);   // quad_perm [1,0,3,2]
             if (lp == 2) rank += (uint32_t)dpp_i<0x4E>(0, (int)rank);   // quad_perm [2,3,0,1]
             if (p == 0 && kc < ng) {
                 sm.u.fc.gsorted[rank] = x;
@@ -1462,7 +1510,7 @@ __device__ __forceinline__ bool nuc_select_fin(const SampleArgs& a, uint32_t row
 #pragma unroll
             for (int c = 0; c < 4; ++c) {
                 const uint32_t i = 4u * (uint32_t)lane + (uint32_t)c;
-                run += i < ng ? g_nuc.u.fc.gw[i] : 0.0;
+                run += i < ng ? g_fin.u.fc.gw[i] : 0.0;
                 pre[c] = run;
             }
             const double incl = wave_scan_incl(run);
@@ -1480,15 +1528,15 @@ __device__ __forceinline__ bool nuc_select_fin(const SampleArgs& a, uint32_t row
                 double pa = 0.0;
 #pragma unroll
                 for (int c = 0; c < 4; ++c) pa = (uint32_t)c == first ? base + pre[c] : pa;
-                g_nuc.l.fp_pos = bal ? 4u * (uint32_t)L + first : kNone;
-                g_nuc.l.fp_m = pa;
+                g_fin.l.fp_pos = bal ? 4u * (uint32_t)L + first : kNone;
+                g_fin.l.fp_m = pa;
             }
         }
         __syncthreads();
         // (the next writer of fp_pos / fp_m is a later first_prefix, after
         // a gather's barriers)
-        p_at = g_nuc.l.fp_m;
-        return g_nuc.l.fp_pos;
+        p_at = g_fin.l.fp_m;
+        return g_fin.l.fp_pos;
     };
 
     // The decision inside range k's sub-bins [s0, s1]: the first position i
@@ -1510,18 +1558,18 @@ __device__ __forceinline__ bool nuc_select_fin(const SampleArgs& a, uint32_t row
                 ng = kNone;
                 return kNone;
             }
-            m = nuc_large_group(k * kNucSub + s0, k * kNucSub + s1, n, list, maxl, inv_t, tgt);
+            m = nuc_large_group(k * kNucSub + s0, k * kNucSub + s1, ng, n, list, maxl, inv_t, tgt);
             if (m == kNone) {
                 ng = kNone;
                 return kNone;
             }
-            gcb = g_nuc.l.lg_cb;
-            gmb = g_nuc.l.lg_mb;
+            gcb = g_fin.l.lg_cb;
+            gmb = g_fin.l.lg_mb;
         }
         const uint32_t pos = first_prefix(m, [&](uint32_t i, double pi) { return hit(gcb + i, gmb + pi); }, p_at);
         if (pos == kNone) return kNone;
         p_at += gmb;
-        key = g_nuc.u.fc.gsorted[pos];
+        key = g_fin.u.fc.gsorted[pos];
         return gcb + pos;
     };
 
@@ -1606,7 +1654,7 @@ __device__ __forceinline__ bool nuc_select_fin(const SampleArgs& a, uint32_t row
             uint32_t cnt = 0;
             double ms = 0.0;
             uint64_t kl = 0ull;
-            for (uint32_t i = tid; i < n; i += NT) {
+            for (uint32_t i = tid; i < n; i += kFT) {
                 const uint32_t c = g_code[i];
                 if (c != kNoCode && c / kNucSub == km) {
                     const uint64_t key = key_at(i);
@@ -1618,9 +1666,9 @@ __device__ __forceinline__ bool nuc_select_fin(const SampleArgs& a, uint32_t row
                     }
                 }
             }
-            const uint32_t tc = block_sum_u<NT>(cnt, sm.l.nall);
-            const double tm = block_sum<NT>(ms, sm.l.sraw);
-            const uint64_t tk = ~block_min_u64<NT>(~kl, sm.l.ck);
+            const uint32_t tc = block_sum_u<kFT>(cnt, sm.l.nall);
+            const double tm = block_sum<kFT>(ms, sm.l.sraw);
+            const uint64_t tk = ~block_min_u64<kFT>(~kl, sm.l.ck);
             keep_m = max(1u, rgl[km].c0 + tc);
             mass_m = rgl[km].m0 + tm;
             key_m = tc > 0 ? tk : ~0ull;
@@ -1868,8 +1916,8 @@ __global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(4))) void nu
 // exact path for a row the plan could not serve, else the exact decisions
 // over the compacted ranges.
 template <int G>
-__global__ __launch_bounds__(NT) void nuc_select_fin_kernel(SampleArgs a) {
-    NucSmem& sm = g_nuc;
+__global__ __launch_bounds__(kFT) void nuc_select_fin_kernel(SampleArgs a) {
+    NucFinSmem& sm = g_fin;
     uint32_t row;
     lcs_params P;
     bool masked;
@@ -1878,7 +1926,7 @@ __global__ __launch_bounds__(NT) void nuc_select_fin_kernel(SampleArgs a) {
     const bool exact = (a.nrow[row - a.nuc_row0].flags & kNucFallback) != 0u;
     if (exact || nuc_select_fin<G>(a, row)) {
         stage_args(&sm.l.args, a);
-        exact_row<kSliceThreads, kFbBins, kFbCap, kFbHistCap, G>(sm.l.args, row, sm.u.ex);
+        exact_row<kFT, kFbBins, kFbCap, kFbHistCap, G>(sm.l.args, row, sm.u.ex);
     }
 }
 
@@ -1895,7 +1943,7 @@ static void launch_passes(const SampleArgs& a, uint32_t nrows, hipStream_t st) {
     hipLaunchKernelGGL(nuc_hist_fin<G>, rgrid, block, 0, st, a);
     hipLaunchKernelGGL(nuc_select<G>, grid, block, 0, st, a.logits, a.row_stride, a.rows, a.slices, a.slice_len,
                        a.vocab, a.nuc_row0, a.all_nucleus, a);
-    hipLaunchKernelGGL(nuc_select_fin_kernel<G>, rgrid, block, 0, st, a);
+    hipLaunchKernelGGL(nuc_select_fin_kernel<G>, rgrid, dim3(kFT), 0, st, a);
 }
 
 hipError_t launch_nucleus(const SampleArgs& a0, hipStream_t st) {
