@@ -21,10 +21,10 @@
 // this kernel's predecessor, 64 rows x 256 columns with the weight fragments
 // loaded straight into registers and the shared x behind a barrier per step):
 //   rows x columns x hidden       before   now
-//   64   x 128256 x 4096 (logits)   217    203
+//   64   x 128256 x 4096 (logits)   218    198
 //   8    x 32000  x 4096            124     51
 //   128  x 128256 x 4096            448    220
-//   1024 x 128256 x 4096           2629    975
+//   1024 x 128256 x 4096           2619    886
 #include <hip/hip_runtime.h>
 #include <math.h>
 #include <stdint.h>
@@ -39,8 +39,6 @@ typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
 typedef float f32x16 __attribute__((ext_vector_type(16)));
 constexpr int kLmThreads = 256;
 constexpr float kL2E = 1.4426950408889634f;
-constexpr int kTK = 32;                       // k per LDS stage
-constexpr uint32_t kTRowB = kTK * 2;          // bytes of a row in a stage
 constexpr uint32_t kBigHidden = 1u << 22;     // above: 64-bit row offsets
 
 // Waits until at most N vector memory operations are outstanding (and every
@@ -76,18 +74,24 @@ __device__ __forceinline__ void block_sync() {
 
 // A workgroup computes 64 VT columns of BR rows, transposed (columns on the
 // MFMA's row side, so that a lane holds many columns of one row and the
-// epilogue reduces in registers): four waves of 32 VT columns x BR / 2 rows in
+// epilogue reduces in registers): NW waves, two over the rows, in
 // v_mfma_f32_32x32x16_bf16 tiles (lane l carries 8 consecutive k of row l % 32
 // of either operand, k chunk l / 32, and returns rows 8 (e / 4) + 4 (l / 32) +
-// e % 4 of column l % 32).
+// e % 4 of column l % 32). The 256 x 256 tile takes eight waves, so that two
+// share a SIMD and one's loads, barriers and epilogue leave the matrix cores to
+// the other (1024 rows: 990 us with four, 963 with eight).
 //
-// Both operands go straight from memory into a ring of ST LDS stages of 32 k
-// with 16-byte DMA loads, so that no register holds data in flight and ST - 1
-// stages are (a stage is 64 bytes of each row). A row's four 16-byte chunks are
-// permuted by bits 2-3 of the row: a fragment read's 16 lanes of a phase then
-// cover the 64 banks once (0 conflict cycles of 67 M; permuted by bits 1-2,
-// half of 133 M). One barrier per stage, in the middle of its products: each
-// wave has then read the stage and its loads of the next one have landed.
+// Both operands go straight from memory into a ring of ST LDS stages of 16 KS k
+// with 16-byte DMA loads, so that no register holds data in flight. The loads
+// are what holds the matrix cores up (without them in the loop 786 us): a
+// stage of 64 k reads whole 128-byte lines, half the requests of 32 k, and two
+// such stages serve as well as four (1024 rows 963 -> 921 us, 64 rows 209 ->
+// 199); narrow and 128-row tiles have too few bytes in flight then (8 x 32000
+// 52 -> 69 us, 128 rows 218 -> 229) and keep 32 k. A row's 16-byte chunks are
+// permuted by its bits from kSw up: a fragment read's 16 lanes of a phase then
+// cover the 64 banks once (0 conflict cycles of 67 M; a bit lower, half of 133
+// M). One barrier per stage, ahead of its last products: each wave has then
+// read the stage and its loads of the next one have landed.
 //
 // The workgroups of a column block are placed on one XCD in consecutive
 // dispatch slots (workgroups are dealt to the 8 XCDs in turn): they run
@@ -97,12 +101,20 @@ __device__ __forceinline__ void block_sync() {
 // offset of their rows (72 rows x 128256 x 4096: 245 -> 225 us); with more the
 // row tiles share x through the L2 by running in step (1024 rows: 1013 against
 // 1057 us with a start of its own).
-template <int VT, int BR, int ST, bool BIG = false>
-__global__ __launch_bounds__(kLmThreads, VT * BR == 1024 ? 1 : 2) void lmhead_tile(LmArgs a) {
+template <int VT, int BR, int ST, int NW = 4, int KS = 2, bool BIG = false>
+__global__ __launch_bounds__(NW * kWave, NW == 8 ? 2 : VT * BR == 1024 ? 1 : 2) void lmhead_tile(LmArgs a) {
     constexpr uint32_t kTV = 64u * VT;        // columns per workgroup
+    constexpr int kTK = 16 * KS;              // k per LDS stage
+    constexpr uint32_t kTRowB = kTK * 2;      // bytes of a row in a stage
     constexpr uint32_t kStage = (kTV + BR) * kTRowB;
-    constexpr int RT = BR / 64;               // 32-row tiles per wave
-    constexpr int LA = kTV / 64, LB = BR / 64;   // DMA loads per wave and stage
+    constexpr int WM = NW / 2;                // waves side by side over the columns, two over the rows
+    constexpr int CT = 2 * VT / WM, RT = BR / 64;   // 32-column and 32-row tiles per wave
+    constexpr uint32_t kCh = 2 * KS, kLog = KS == 4 ? 3 : 2;   // 16-byte chunks of a row
+    constexpr uint32_t kSw = KS == 4 ? 1 : 2;   // the row bits that permute them start here
+    constexpr int kLR = 64 / (int)kCh * NW;   // rows that one DMA load of every wave covers
+    constexpr int LA = kTV / kLR, LB = BR / kLR;   // DMA loads per wave and stage
+    static_assert(KS == 2 || (KS == 4 && ST == 2), "the schedule of the k-loop");
+    static_assert(LA * kLR == (int)kTV && LB * kLR == BR && CT * WM == 2 * VT, "tile shape");
     constexpr int LPS = LA + LB;
     __shared__ __attribute__((aligned(128))) unsigned char lds[ST * kStage];
     const uint32_t tid = tid_x();
@@ -115,22 +127,22 @@ __global__ __launch_bounds__(kLmThreads, VT * BR == 1024 ? 1 : 2) void lmhead_ti
     const uint32_t K = a.hidden, V = a.vocab;
     const uint32_t n0 = nb * kTV;
     const uint32_t vrows = min((uint32_t)BR, a.rows - r0), vcols = min(kTV, V - n0);
-    const uint32_t wm = (uint32_t)wv & 1u, wn = (uint32_t)wv >> 1;   // the wave's columns and rows
+    const uint32_t wm = (uint32_t)wv % WM, wn = (uint32_t)wv / WM;   // the wave's columns and rows
     const uint16_t* wbase = a.w + (uint64_t)n0 * K;
     const uint16_t* xbase = a.x + (uint64_t)r0 * K;
     const __amdgpu_buffer_rsrc_t wrs =
         __builtin_amdgcn_make_buffer_rsrc(const_cast<uint16_t*>(wbase), 0, (int)(vcols * K * 2u), 0x00020000);
     const __amdgpu_buffer_rsrc_t xrs =
         __builtin_amdgcn_make_buffer_rsrc(const_cast<uint16_t*>(xbase), 0, (int)(vrows * K * 2u), 0x00020000);
-    // DMA load i of a wave covers rows 64 i + 16 wv + lane / 4, a 16-byte
+    // DMA load i of a wave covers rows kLR i + 16 wv + lane / 4, a 16-byte
     // chunk per lane; rows past the tile read row 0 (masked in the epilogue)
-    const uint32_t rr = 16u * (uint32_t)wv + ((uint32_t)lane >> 2);
-    const uint32_t ch = (((uint32_t)lane & 3u) ^ ((rr >> 2) & 3u)) * 16u;
+    const uint32_t rr = kWave / kCh * (uint32_t)wv + ((uint32_t)lane >> kLog);
+    const uint32_t ch = (((uint32_t)lane & (kCh - 1u)) ^ ((rr >> kSw) & (kCh - 1u))) * 16u;
     uint32_t wo[LA], xo[LB];
 #pragma unroll
-    for (int i = 0; i < LA; ++i) wo[i] = (64u * i + rr < vcols ? 64u * i + rr : 0u) * K * 2u + ch;
+    for (int i = 0; i < LA; ++i) wo[i] = (kLR * i + rr < vcols ? kLR * i + rr : 0u) * K * 2u + ch;
 #pragma unroll
-    for (int i = 0; i < LB; ++i) xo[i] = (64u * i + rr < vrows ? 64u * i + rr : 0u) * K * 2u + ch;
+    for (int i = 0; i < LB; ++i) xo[i] = (kLR * i + rr < vrows ? kLR * i + rr : 0u) * K * 2u + ch;
     const uint32_t nsteps = K / kTK;
     const uint32_t rot = a.nchunks == 1u ? nb % nsteps : 0u;
     // (the byte offset of stage t in a row; stages past the end re-read the last)
@@ -139,9 +151,9 @@ __global__ __launch_bounds__(kLmThreads, VT * BR == 1024 ? 1 : 2) void lmhead_ti
         return (q >= nsteps ? q - nsteps : q) * kTRowB;
     };
     auto issue1 = [&](int i, uint32_t ko, uint32_t sl) {   // DMA load i of a stage
-        unsigned char* b = lds + sl * kStage + (uint32_t)wv * 1024u + i * 4096;
+        unsigned char* b = lds + sl * kStage + (uint32_t)wv * 1024u + i * (kLR * kTRowB);
         if (BIG) {   // (the row offsets need 64 bits)
-            const uint32_t r = 64u * (uint32_t)(i < LA ? i : i - LA) + rr;
+            const uint32_t r = kLR * (uint32_t)(i < LA ? i : i - LA) + rr;
             const uint16_t* p = i < LA ? wbase + (uint64_t)(r < vcols ? r : 0u) * K : xbase + (uint64_t)(r < vrows ? r : 0u) * K;
             dma16_at(reinterpret_cast<const unsigned char*>(p) + ko + ch, b);
         } else if (i < LA) {
@@ -154,23 +166,23 @@ __global__ __launch_bounds__(kLmThreads, VT * BR == 1024 ? 1 : 2) void lmhead_ti
 #pragma unroll
         for (int i = 0; i < LPS; ++i) issue1(i, koff(t), sl);
     };
-    f32x16 acc[VT][RT];
+    f32x16 acc[CT][RT];
 #pragma unroll
-    for (int i = 0; i < VT; ++i)
+    for (int i = 0; i < CT; ++i)
 #pragma unroll
         for (int j = 0; j < RT; ++j)
 #pragma unroll
             for (int e = 0; e < 16; ++e) acc[i][j][e] = 0.0f;
     // fragment s (16 k) of row r: chunk 2 s + lane / 32
     const uint32_t lr = (uint32_t)lane & 31u, lh = (uint32_t)lane >> 5;
-    uint32_t fo[2];
+    uint32_t fo[KS];
 #pragma unroll
-    for (uint32_t s = 0; s < 2; ++s) fo[s] = lr * kTRowB + (((2u * s + lh) ^ ((lr >> 2) & 3u)) * 16u);
-    struct Frag { bf16x8 w[VT], x[RT]; };
+    for (uint32_t s = 0; s < KS; ++s) fo[s] = lr * kTRowB + (((2u * s + lh) ^ ((lr >> kSw) & (kCh - 1u))) * 16u);
+    struct Frag { bf16x8 w[CT], x[RT]; };
     // read i of a fragment set: x first (every product needs all of it), then w
-    constexpr int NR = VT + RT, NP = VT * RT;
+    constexpr int NR = CT + RT, NP = CT * RT;
     auto read1 = [&](Frag& f, int i, uint32_t sl, int s) {
-        const unsigned char* pw = lds + sl * kStage + wm * (kTV / 2 * kTRowB) + fo[s];
+        const unsigned char* pw = lds + sl * kStage + wm * (kTV / WM * kTRowB) + fo[s];
         const unsigned char* px = lds + sl * kStage + kTV * kTRowB + wn * (BR / 2 * kTRowB) + fo[s];
         if (i < RT) f.x[i < RT ? i : 0] = *reinterpret_cast<const bf16x8*>(px + i * 32 * kTRowB);
         else f.w[i >= RT ? i - RT : 0] = *reinterpret_cast<const bf16x8*>(pw + (i - RT) * 32 * kTRowB);
@@ -189,27 +201,39 @@ __global__ __launch_bounds__(kLmThreads, VT * BR == 1024 ? 1 : 2) void lmhead_ti
     uint32_t sl = 0u;
     // Every LDS read and DMA load is issued behind a product: a wave issues
     // in order, and eight DMA loads in a row hold it for longer than the
-    // products queued ahead of them last (1024 rows: 1022 -> 980 us).
+    // products queued ahead of them last (1024 rows, four waves: 1022 -> 980 us).
+    // (KS 4, two stages: half of a stage's loads go out behind the last products
+    // of the stage whose place it takes, half behind the next stage's first)
+    uint32_t kn = 0u;   // the offset of the stage whose second half is to be issued
     for (uint32_t t = 0; t < nsteps; ++t) {
         const uint32_t ns = sl + 1u == (uint32_t)ST ? 0u : sl + 1u;
+        constexpr int H = LPS / 2;
 #pragma unroll
-        for (int k = 0; k < NP; ++k) {
-            mul1(f0, k);
+        for (int s = 0; s < KS - 1; ++s) {
+            const bool more = KS == 4 && s == 0;
 #pragma unroll
-            for (int i = k * NR / NP; i < (k + 1) * NR / NP; ++i) read1(f1, i, sl, 1);
-            __builtin_amdgcn_sched_barrier(0);
+            for (int k = 0; k < NP; ++k) {
+                mul1(s % 2 == 0 ? f0 : f1, k);
+#pragma unroll
+                for (int i = k * (NR + (more ? LPS - H : 0)) / NP; i < (k + 1) * (NR + (more ? LPS - H : 0)) / NP; ++i) {
+                    if (i < NR) read1(s % 2 == 0 ? f1 : f0, i, sl, s + 1);
+                    else if (t != 0u) issue1(H + i - NR, kn, ns);
+                }
+                __builtin_amdgcn_sched_barrier(0);
+            }
         }
         // stage t is read, stage t + 1 has landed, in every wave
-        wait_vm_lgkm<(ST - 2) * LPS>();
+        wait_vm_lgkm<KS == 4 ? 0 : (ST - 2) * LPS>();
         block_sync();
-        const uint32_t ko = koff(t + ST);
+        kn = koff(t + ST);
+        constexpr int L = KS == 4 ? H : LPS;
 #pragma unroll
         for (int k = 0; k < NP; ++k) {
             mul1(f1, k);
 #pragma unroll
-            for (int i = k * (NR + LPS) / NP; i < (k + 1) * (NR + LPS) / NP; ++i) {
+            for (int i = k * (NR + L) / NP; i < (k + 1) * (NR + L) / NP; ++i) {
                 if (i < NR) read1(f0, i, ns, 0);
-                else issue1(i - NR, ko, sl);
+                else issue1(i - NR, kn, sl);
             }
             __builtin_amdgcn_sched_barrier(0);
         }
@@ -218,21 +242,21 @@ __global__ __launch_bounds__(kLmThreads, VT * BR == 1024 ? 1 : 2) void lmhead_ti
     wait_vm_lgkm<0>();
     __syncthreads();   // (the last loads have landed: the ring is free)
 
-    // ---- epilogue: acc[i][j][e] is column n0 + kTV / 2 wm + 32 i + 8 (e / 4) +
+    // ---- epilogue: acc[i][j][e] is column n0 + kTV / WM wm + 32 i + 8 (e / 4) +
     // 4 lh + e % 4 of row r0 + BR / 2 wn + 32 j + lr ----
     struct Part { float max, sum, draft; uint32_t idx; };
-    Part* part = reinterpret_cast<Part*>(lds);   // [2][BR]: by the wave's columns
+    Part* part = reinterpret_cast<Part*>(lds);   // [WM][BR]: by the wave's columns
     const bool full = vcols == kTV;
     const bool vec = a.logits && (a.ld_logits & 3u) == 0u && (reinterpret_cast<uintptr_t>(a.logits) & 15u) == 0u;
 #pragma unroll
     for (int j = 0; j < RT; ++j) {
         const uint32_t rl = wn * (BR / 2) + 32u * j + lr;   // the lane's row in the tile
         const bool rin = rl < vrows;
-        const uint32_t cb = kTV / 2 * wm + 4u * lh;            // columns cb + 32 i + 8 (e / 4) + e % 4
+        const uint32_t cb = kTV / WM * wm + 4u * lh;            // columns cb + 32 i + 8 (e / 4) + e % 4
         if (a.logits && rin) {
             float* out = a.logits + (uint64_t)(r0 + rl) * a.ld_logits + n0;
 #pragma unroll
-            for (int i = 0; i < VT; ++i)
+            for (int i = 0; i < CT; ++i)
 #pragma unroll
                 for (int q = 0; q < 4; ++q) {
                     const uint32_t c = cb + 32u * i + 8u * q;
@@ -249,7 +273,7 @@ __global__ __launch_bounds__(kLmThreads, VT * BR == 1024 ? 1 : 2) void lmhead_ti
         const float NEG = -__builtin_huge_valf();
         if (!full) {
 #pragma unroll
-            for (int i = 0; i < VT; ++i)
+            for (int i = 0; i < CT; ++i)
 #pragma unroll
                 for (int e = 0; e < 16; ++e)
                     if (cb + 32u * i + 8u * (e / 4) + e % 4 >= vcols) acc[i][j][e] = NEG;
@@ -257,7 +281,7 @@ __global__ __launch_bounds__(kLmThreads, VT * BR == 1024 ? 1 : 2) void lmhead_ti
         // the lane's max, its first column, the draft's logit
         float m = acc[0][j][0];
 #pragma unroll
-        for (int i = 0; i < VT; ++i)
+        for (int i = 0; i < CT; ++i)
 #pragma unroll
             for (int e = 0; e < 16; ++e) m = fmaxf(m, acc[i][j][e]);
         const int32_t dr = a.draft && rin ? a.draft[r0 + rl] : -1;
@@ -265,16 +289,16 @@ __global__ __launch_bounds__(kLmThreads, VT * BR == 1024 ? 1 : 2) void lmhead_ti
         uint32_t ci = kTV;
         float dl = 0.0f;
 #pragma unroll
-        for (int i = VT - 1; i >= 0; --i)
+        for (int i = CT - 1; i >= 0; --i)
 #pragma unroll
             for (int e = 15; e >= 0; --e) {
                 const uint32_t c = 32u * i + 8u * (e / 4) + e % 4;
                 ci = acc[i][j][e] == m ? c : ci;
             }
         uint32_t found = 0u;
-        if (ballot(dc < kTV / 2 && (dc & 4u) == 0u) != 0u) {
+        if (ballot(dc < kTV / WM && (dc & 4u) == 0u) != 0u) {
 #pragma unroll
-            for (int i = 0; i < VT; ++i)
+            for (int i = 0; i < CT; ++i)
 #pragma unroll
                 for (int e = 0; e < 16; ++e) {
                     const uint32_t c = 32u * i + 8u * (e / 4) + e % 4;
@@ -285,7 +309,7 @@ __global__ __launch_bounds__(kLmThreads, VT * BR == 1024 ? 1 : 2) void lmhead_ti
         // (a lane whose columns all lie past the vocabulary: max -inf, no term)
         float s = 0.0f;
 #pragma unroll
-        for (int i = 0; i < VT; ++i)
+        for (int i = 0; i < CT; ++i)
 #pragma unroll
             for (int e = 0; e < 16; e += 4) {
                 float t[4];
@@ -305,16 +329,25 @@ __global__ __launch_bounds__(kLmThreads, VT * BR == 1024 ? 1 : 2) void lmhead_ti
     }
     __syncthreads();
     if (tid < vrows) {
-        const Part p = part[tid], q = part[BR + tid];
         const float NEG = -__builtin_huge_valf();
-        const float M = fmaxf(p.max, q.max);
+        Part p = part[tid];
+#pragma unroll
+        for (int w = 1; w < WM; ++w) {
+            // (equal maxima: the lower columns are p's; columns past the
+            // vocabulary: max -inf)
+            const Part q = part[w * BR + tid];
+            const float M = fmaxf(p.max, q.max);
+            p.sum = p.sum * __builtin_amdgcn_exp2f((p.max - M) * kL2E) +
+                    (q.max == NEG ? 0.0f : q.sum * __builtin_amdgcn_exp2f((q.max - M) * kL2E));
+            p.draft = (p.idx & kLmDraftBit) ? p.draft : q.draft;
+            p.idx = ((p.max >= q.max ? p.idx : q.idx) & ~kLmDraftBit) | ((p.idx | q.idx) & kLmDraftBit);
+            p.max = M;
+        }
         LmRec rec;
-        rec.max = M;
-        // (equal maxima: the lower columns are p's)
-        rec.idx = (n0 + ((p.max >= q.max ? p.idx : q.idx) & ~kLmDraftBit)) | ((p.idx | q.idx) & kLmDraftBit);
-        rec.sum = p.sum * __builtin_amdgcn_exp2f((p.max - M) * kL2E) +
-                  (q.max == NEG ? 0.0f : q.sum * __builtin_amdgcn_exp2f((q.max - M) * kL2E));
-        rec.draft = (p.idx & kLmDraftBit) ? p.draft : q.draft;
+        rec.max = p.max;
+        rec.idx = n0 + p.idx;   // (the draft bit is bit 31)
+        rec.sum = p.sum;
+        rec.draft = p.draft;
         a.recs[(uint64_t)(r0 + tid) * a.nblocks + nb] = rec;
     }
 }
@@ -426,16 +459,16 @@ hipError_t launch_lmhead(const LmArgs& a0, uint32_t cus, hipStream_t st) {
     a.nchunks = (a.rows + sh.br - 1u) / sh.br;
     const dim3 grid(8u * ((a.nblocks + 7u) / 8u) * a.nchunks), block(kLmThreads);
     // (stages: as deep as two workgroups a CU leave room for, or one where
-    // there is no second; two where two 256-column tiles a CU are all there
-    // is: 209 against 212 us)
-    if (a.hidden > kBigHidden) hipLaunchKernelGGL((lmhead_tile<4, 64, 3, true>), grid, block, 0, st, a);
-    else if (sh.br == 256u && sh.vt == 4u) hipLaunchKernelGGL((lmhead_tile<4, 256, 4>), grid, block, 0, st, a);
+    // there is no second; two of 64 k where two 256-column tiles a CU are all
+    // there is: 199 us against 209 with two of 32 k and 212 with three)
+    if (a.hidden > kBigHidden) hipLaunchKernelGGL((lmhead_tile<4, 64, 3, 4, 2, true>), grid, block, 0, st, a);
+    else if (sh.br == 256u && sh.vt == 4u) hipLaunchKernelGGL((lmhead_tile<4, 256, 2, 8, 4>), grid, dim3(8 * kWave), 0, st, a);
     else if (sh.br == 256u) hipLaunchKernelGGL((lmhead_tile<2, 256, 3>), grid, block, 0, st, a);
     else if (sh.br == 128u && sh.vt == 4u) hipLaunchKernelGGL((lmhead_tile<4, 128, 3>), grid, block, 0, st, a);
     else if (sh.br == 128u) hipLaunchKernelGGL((lmhead_tile<2, 128, 4>), grid, block, 0, st, a);
     else if (sh.vt == 5u) hipLaunchKernelGGL((lmhead_tile<5, 64, 3>), grid, block, 0, st, a);
     else if (sh.vt == 4u && a.nblocks > cus && a.nblocks <= 2u * cus)
-        hipLaunchKernelGGL((lmhead_tile<4, 64, 2>), grid, block, 0, st, a);
+        hipLaunchKernelGGL((lmhead_tile<4, 64, 2, 4, 4>), grid, block, 0, st, a);
     else if (sh.vt == 4u) hipLaunchKernelGGL((lmhead_tile<4, 64, 4>), grid, block, 0, st, a);
     else if (sh.vt == 2u) hipLaunchKernelGGL((lmhead_tile<2, 64, 4>), grid, block, 0, st, a);
     else hipLaunchKernelGGL((lmhead_tile<1, 64, 6>), grid, block, 0, st, a);
