@@ -33,7 +33,7 @@ MALL_BYTES = 256 << 20
 # pattern (SQL LIKE) matching them, and the stem of their profile summaries
 # ("a|b" matches either)
 KERNEL = {"c1g": ("slice_stats|row_fin", "sliced"), "c1s": ("slice_stats|row_fin", "sliced"),
-          "c2": ("slice_stats|row_fin", "sliced"), "c2w": ("slice_stats|row_fin", "sliced"),
+          "c2": ("slice_stats|row_fin", "sliced"), "c2w": ("slice_stats|row_fin|nuc_", "sliced"),
           "c3": ("nuc_", "nucleus"),
           "c4": ("nuc_", "nucleus"), "c5": ("verify_kernel|accept_kernel", "verify")}
 
@@ -389,6 +389,8 @@ def exact_clocks(workload: str, rows: int | None, calls: int = 8):
     L.lcs_xprof_read.argtypes = [C.c_void_p, C.c_void_p]
     L.lcs_xprof_clear.restype = C.c_int
     w = W.make(workload, rows=rows)
+    if workload == "c2w":   # (with c2w's own cuts row_fin hands its rows to the nucleus kernels)
+        w.params["temperature"], w.params["min_p"] = 1.0, 0.05
     s = SM.Sampler(device=0, max_rows=w.rows, max_vocab=262144, max_hist=4096, max_top=20)
     d = s.upload(w)
     run = s.prepare(d, s.alloc_out(w.rows, w.n_top, w.want_logprobs, diag=False))

@@ -103,15 +103,14 @@ __global__ __launch_bounds__(kDraftThreads) void ngram_draft_kernel(DraftArgs a)
 }
 
 // Threads per sequence: the contexts' lengths are known on the device only, so
-// the number of sequences decides: a CU each, 1024 threads; above, 512, two a
-// CU (us a call with 256 / 512 / 1024 threads, contexts up to 32768 tokens: 64
-// sequences 12.1 / 8.2 / 7.2, 256: 14.2 / 9.1 / 7.5, 512: 17.2 / 12.6 / 13.7; up
-// to 131072 tokens, one sequence 11.3 / 8.1 / 7.5, 512: 57 / 39 / 33; 512 of up
-// to 4096: 6.0 / 6.1 / 7.9). Above 1024 sequences the small workgroups share
-// the CUs as they are.
+// the number of sequences decides. Up to one a CU, 512 threads (us a call with
+// 256 / 512 / 1024 threads, contexts up to 32768 tokens: 64 sequences 12.1 / 8.2
+// / 7.2, 256: 14.2 / 9.1 / 7.5; one of up to 131072 tokens 11.3 / 8.1 / 7.5;
+// the kernel alone on contexts up to 4096, 64 sequences: 3.9 / 4.1 / 4.9: a
+// larger workgroup starts later). Above, 256 (512 contexts of 4096 tokens: 4.1
+// / 4.8; long ones would gain, up to 32768 tokens 17.2 / 12.6).
 hipError_t launch_draft(const DraftArgs& a, hipStream_t st) {
-    if (a.n_seq <= 256u) hipLaunchKernelGGL(ngram_draft_kernel<1024>, dim3(a.n_seq), dim3(1024), 0, st, a);
-    else if (a.n_seq <= 1024u) hipLaunchKernelGGL(ngram_draft_kernel<512>, dim3(a.n_seq), dim3(512), 0, st, a);
+    if (a.n_seq <= 256u) hipLaunchKernelGGL(ngram_draft_kernel<512>, dim3(a.n_seq), dim3(512), 0, st, a);
     else hipLaunchKernelGGL(ngram_draft_kernel<256>, dim3(a.n_seq), dim3(256), 0, st, a);
     return hipGetLastError();
 }

@@ -103,7 +103,7 @@ def test_draft_rejects_bad_arguments(sampler):
 
 
 @pytest.mark.gpu
-@pytest.mark.parametrize("n_seq,chunk", [(3, 16384), (256, 16384), (257, 8192), (1025, 4096)])
+@pytest.mark.parametrize("n_seq,chunk", [(3, 8192), (256, 8192), (257, 4096)])
 def test_draft_workgroup_sizes(sampler, n_seq, chunk):
     """Each workgroup size at the edges of its rounds (16 starts a thread): the
     only match one start before, at and after a round's border, the first
