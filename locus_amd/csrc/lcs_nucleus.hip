@@ -1,7 +1,7 @@
 // Nucleus path for MI355X (gfx950): stochastic rows whose candidate set
-// stays large (top-p only, constrained rows, min-p over a flat row, top-k
-// beyond the sliced top-k path), in three slice-parallel passes over
-// device-resident logits.
+// stays large (top-p only, constrained rows, top-k beyond the sliced top-k
+// path, and min-p rows whose windows row_fin found too wide), in three
+// slice-parallel passes over device-resident logits.
 //
 // Each pass cuts a row into `slices` workgroups of 256 threads (one HBM read
 // of <= 8192 logits each, 32 per thread in registers), as the sliced kernel

@@ -18,7 +18,9 @@
 //   logprobs, argmax, or the window / top-k walk top-p -> min-p -> draw with
 //   exact f64 weights. A row whose decision the records cannot settle (a
 //   window or list overflow, a top-p decision within the normaliser's error
-//   bound) is resolved there by exact_row, the single-workgroup exact path.
+//   bound) is handed to the nucleus kernels when they follow in the call (min-p
+//   window rows), else resolved there by exact_row, the single-workgroup exact
+//   path.
 //
 // No workgroup waits on or signals another, so the path needs no
 // cross-workgroup memory ordering inside a kernel.

@@ -13,8 +13,8 @@ Configurations (seed base ``S = 20261200 + n`` for configuration n):
   through a seeded permutation; repeat 1.1, frequency 0.5, presence 0.3,
   repeat_last_n 2048; T=0.7, min_p 0.05, top_p 0.9; top-5 logprobs.
 * ``c2w`` - ``c2`` with N(0, 1) logits, T=1.5 and min_p 0.01: min-p windows
-  of thousands of ids, past a slice's window record, so every row takes the
-  exact path inside the row finalize (a stress case, not a BASELINE config).
+  of thousands of ids, past a slice's window record, so the row finalize hands
+  every row to the nucleus kernels (a stress case).
 * ``c3`` - B=256, V=151936 f32 ~ N(0, 1); T=1.5, top_p 0.98.
 * ``c4`` - B=32, V=128256 f32 ~ N(0, 2.5^2); per-row allow mask of V/32
   words with log-uniform density in [5e-4, 0.3] built from runs of 1..64 ids;
