@@ -345,7 +345,9 @@ __global__ __launch_bounds__(NW * kWave, NW == 8 ? 2 : VT * BR == 1024 ? 1 : 2) 
         }
         LmRec rec;
         rec.max = p.max;
-        rec.idx = n0 + p.idx;   // (the draft bit is bit 31)
+        // (a block of NaNs has no column that equals its max: its first one)
+        const uint32_t col = p.idx & ~kLmDraftBit;
+        rec.idx = (n0 + (col < vcols ? col : 0u)) | (p.idx & kLmDraftBit);
         rec.sum = p.sum;
         rec.draft = p.draft;
         a.recs[(uint64_t)(r0 + tid) * a.nblocks + nb] = rec;

@@ -149,6 +149,25 @@ def test_row_tiles_are_exact(sampler, rows, vocab, hidden):
         assert np.array_equal(h[k], g[k]) and np.array_equal(out[k].cpu().numpy(), g[k]), k
 
 
+@pytest.mark.parametrize("rows,vocab", [(3, 1), (5, 70), (64, 300), (130, 513)])
+def test_argmax_stays_in_range_for_nan_and_inf(sampler, rows, vocab):
+    """Rows of NaN, of -inf and with one +inf: the argmax is an id of the
+    vocabulary (a decode loop looks up its embedding)."""
+    torch = sampler.torch
+    hidden = 64
+    x = torch.ones((rows, hidden), dtype=torch.bfloat16, device="cuda")
+    w = torch.ones((vocab, hidden), dtype=torch.bfloat16, device="cuda")
+    x[0] = float("nan")
+    x[1] = float("-inf")
+    x[2, 0] = float("inf")
+    g = run(sampler, x, w)
+    assert ((g["argmax_ids"] >= 0) & (g["argmax_ids"] < vocab)).all(), g["argmax_ids"]
+    assert (g["argmax_ids"][3:] == 0).all()
+    w[vocab // 2:] = float("nan")
+    g = run(sampler, x, w)
+    assert ((g["argmax_ids"] >= 0) & (g["argmax_ids"] < vocab)).all(), g["argmax_ids"]
+
+
 @pytest.mark.parametrize("vocab", [20000, 140000])
 def test_drafts_and_acceptance(sampler, vocab):
     """rows_per_seq = 8: each sequence's drafts agree with the argmax on a
