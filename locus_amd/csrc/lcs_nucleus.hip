@@ -1249,9 +1249,10 @@ __device__ __attribute__((noinline)) uint32_t nuc_large_group(uint32_t c0, uint3
         glo = kmin + ((uint64_t)b0 << sh);
         ghi = b1 >= lastb ? kmax : kmin + (((uint64_t)b1 + 1u) << sh) - 1u;
     }
-    if (m > kGroupMax) return kNone;
+    if (m > kGroupMax) return kNone;   // (uniform)
+    __syncthreads();   // (every wave has formed m: lg_n is free)
     if (tid == 0) sm.l.lg_n = 0u;
-    __syncthreads();   // (the buckets are read, lg_n is cleared)
+    __syncthreads();
     each([&](uint64_t key) { g_fin.u.fc.gkey[atomicAdd(&g_fin.l.lg_n, 1u)] = key; });
     __syncthreads();
     if (tid < m) {
