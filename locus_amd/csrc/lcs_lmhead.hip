@@ -337,7 +337,7 @@ __global__ __launch_bounds__(NW * kWave, NW == 8 ? 2 : VT * BR == 1024 ? 1 : 2) 
             // vocabulary: max -inf)
             const Part q = part[w * BR + tid];
             const float M = fmaxf(p.max, q.max);
-            p.sum = p.sum * __builtin_amdgcn_exp2f((p.max - M) * kL2E) +
+            p.sum = (p.max == NEG ? 0.0f : p.sum * __builtin_amdgcn_exp2f((p.max - M) * kL2E)) +
                     (q.max == NEG ? 0.0f : q.sum * __builtin_amdgcn_exp2f((q.max - M) * kL2E));
             p.draft = (p.idx & kLmDraftBit) ? p.draft : q.draft;
             p.idx = ((p.max >= q.max ? p.idx : q.idx) & ~kLmDraftBit) | ((p.idx | q.idx) & kLmDraftBit);

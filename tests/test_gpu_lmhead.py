@@ -168,6 +168,25 @@ def test_argmax_stays_in_range_for_nan_and_inf(sampler, rows, vocab):
     assert ((g["argmax_ids"] >= 0) & (g["argmax_ids"] < vocab)).all(), g["argmax_ids"]
 
 
+@pytest.mark.parametrize("rows,vocab", [(5, 300), (64, 1000), (130, 1000), (256, 1000)])
+def test_log_z_of_rows_with_inf_blocks(sampler, rows, vocab):
+    """Columns of -inf, whole blocks of them too, have no weight in log z; a
+    row of nothing but -inf has none (as in logprobs_from, which then divides
+    by the exponential of -inf - -inf)."""
+    torch = sampler.torch
+    x = torch.ones((rows, 64), dtype=torch.bfloat16, device="cuda")
+    for lo, hi in [(0, vocab - 7), (0, vocab // 2), (vocab // 3, vocab), (40, 41), (0, vocab)]:
+        w = torch.from_numpy(np.linspace(-0.1, 0.1, vocab, dtype=np.float32)[:, None].repeat(64, 1)).to(torch.bfloat16).cuda()
+        w[lo:hi] = float("-inf")
+        g = run(sampler, x, w)
+        if (lo, hi) == (0, vocab):
+            assert np.isnan(g["log_z"]).all()
+        else:
+            lz = logsumexp64(g["logits"])
+            assert (np.abs(g["log_z"] - lz) <= LOGPROB_TOL).all(), (lo, hi, g["log_z"][0], lz[0])
+            assert np.array_equal(g["argmax_ids"], np.argmax(g["logits"], axis=1))
+
+
 @pytest.mark.parametrize("vocab", [20000, 140000])
 def test_drafts_and_acceptance(sampler, vocab):
     """rows_per_seq = 8: each sequence's drafts agree with the argmax on a
