@@ -62,6 +62,13 @@ __device__ __forceinline__ void dma16_at(const void* src, unsigned char* dst) {
     __builtin_amdgcn_global_load_lds((const __attribute__((address_space(1))) void*)src,
                                      (__attribute__((address_space(3))) void*)dst, 16, 0, 0);
 }
+// NaN, by its bits: the build's float comparisons and selects assume that there
+// are none (the empty asm keeps the compiler from concluding the same here).
+__device__ __forceinline__ bool nan_bits(float v) {
+    uint32_t u = __float_as_uint(v);
+    asm("" : "+v"(u));
+    return (u & 0x7fffffffu) > 0x7f800000u;
+}
 // A workgroup barrier that waits for no memory operation.
 __device__ __forceinline__ void block_sync() {
     __builtin_amdgcn_sched_barrier(0);
@@ -305,8 +312,6 @@ __global__ __launch_bounds__(NW * kWave, NW == 8 ? 2 : VT * BR == 1024 ? 1 : 2) 
                     if (dc == c) { dl = acc[i][j][e]; found = kLmDraftBit; }
                 }
         }
-        ci += cb;
-        // (a lane whose columns all lie past the vocabulary: max -inf, no term)
         float s = 0.0f;
 #pragma unroll
         for (int i = 0; i < CT; ++i)
@@ -317,13 +322,32 @@ __global__ __launch_bounds__(NW * kWave, NW == 8 ? 2 : VT * BR == 1024 ? 1 : 2) 
                 for (int k = 0; k < 4; ++k) t[k] = __builtin_amdgcn_exp2f((acc[i][j][e + k] - m) * kL2E);
                 s += (t[0] + t[1]) + (t[2] + t[3]);
             }
-        s = m == NEG ? 0.0f : s;
+        if (nan_bits(s)) {
+            // a NaN or +inf, or nothing but -inf (columns past the vocabulary
+            // too): the max and its first column again, NaNs left out, which
+            // keep the sum a NaN; columns of -inf have no term
+            bool nan = false;
+            m = NEG;
+            ci = kTV;
+#pragma unroll
+            for (int i = 0; i < CT; ++i)
+#pragma unroll
+                for (int e = 0; e < 16; ++e) {
+                    const float v = acc[i][j][e];
+                    const bool n = nan_bits(v), up = !n && (ci == kTV || v > m);
+                    nan = nan || n;
+                    m = up ? v : m;
+                    ci = up ? 32u * i + 8u * (e / 4) + e % 4 : ci;
+                }
+            s = m == NEG && !nan ? 0.0f : s;
+        }
+        ci += cb;
         // lanes l and l + 32 share a row
         const float m2 = __shfl_xor(m, 32), s2 = __shfl_xor(s, 32), d2 = __shfl_xor(dl, 32);
         const uint32_t c2 = (uint32_t)__shfl_xor((int)ci, 32), f2 = (uint32_t)__shfl_xor((int)found, 32);
         const float M = fmaxf(m, m2);
-        s = (m == NEG ? 0.0f : s * __builtin_amdgcn_exp2f((m - M) * kL2E)) +
-            (m2 == NEG ? 0.0f : s2 * __builtin_amdgcn_exp2f((m2 - M) * kL2E));
+        s = (m == NEG ? s : s * __builtin_amdgcn_exp2f((m - M) * kL2E)) +
+            (m2 == NEG ? s2 : s2 * __builtin_amdgcn_exp2f((m2 - M) * kL2E));
         ci = m > m2 ? ci : m2 > m ? c2 : min(ci, c2);
         if (lh == 0u) part[wm * BR + rl] = Part{M, s, found ? dl : d2, ci | found | f2};
     }
@@ -333,14 +357,14 @@ __global__ __launch_bounds__(NW * kWave, NW == 8 ? 2 : VT * BR == 1024 ? 1 : 2) 
         Part p = part[tid];
 #pragma unroll
         for (int w = 1; w < WM; ++w) {
-            // (equal maxima: the lower columns are p's; columns past the
-            // vocabulary: max -inf)
+            // (a side of -inf: its sum is 0, or NaN where it holds one)
             const Part q = part[w * BR + tid];
             const float M = fmaxf(p.max, q.max);
-            p.sum = (p.max == NEG ? 0.0f : p.sum * __builtin_amdgcn_exp2f((p.max - M) * kL2E)) +
-                    (q.max == NEG ? 0.0f : q.sum * __builtin_amdgcn_exp2f((q.max - M) * kL2E));
+            p.sum = (p.max == NEG ? p.sum : p.sum * __builtin_amdgcn_exp2f((p.max - M) * kL2E)) +
+                    (q.max == NEG ? q.sum : q.sum * __builtin_amdgcn_exp2f((q.max - M) * kL2E));
             p.draft = (p.idx & kLmDraftBit) ? p.draft : q.draft;
-            p.idx = ((p.max >= q.max ? p.idx : q.idx) & ~kLmDraftBit) | ((p.idx | q.idx) & kLmDraftBit);
+            const uint32_t pc = p.idx & ~kLmDraftBit, qc = q.idx & ~kLmDraftBit;
+            p.idx = (p.max > q.max ? pc : q.max > p.max ? qc : min(pc, qc)) | ((p.idx | q.idx) & kLmDraftBit);
             p.max = M;
         }
         LmRec rec;

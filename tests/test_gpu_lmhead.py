@@ -168,6 +168,25 @@ def test_argmax_stays_in_range_for_nan_and_inf(sampler, rows, vocab):
     assert ((g["argmax_ids"] >= 0) & (g["argmax_ids"] < vocab)).all(), g["argmax_ids"]
 
 
+@pytest.mark.parametrize("rows,vocab", [(3, 64), (5, 300), (64, 1000), (130, 1000), (256, 1000)])
+def test_argmax_beside_nan_columns(sampler, rows, vocab):
+    """Columns of NaN beside finite ones, also all of one wave's or of one
+    block's: the argmax is the first of the greatest finite columns, and log z
+    is NaN (one of the sum's terms is)."""
+    torch = sampler.torch
+    x = torch.ones((rows, 64), dtype=torch.bfloat16, device="cuda")
+    best = vocab // 4 + 3
+    for lo, hi in [(vocab // 2, vocab), (32, 64), (64, 128), (0, vocab // 4), (best - 1, best), (best + 1, best + 2)]:
+        w = torch.full((vocab, 64), -1.0, dtype=torch.bfloat16, device="cuda")
+        w[best:best + 2] = 1.0
+        w[lo:hi] = float("nan")
+        g = run(sampler, x, w)
+        want = np.argmax(np.where(np.isnan(g["logits"]), -np.inf, g["logits"]), axis=1)
+        assert np.array_equal(g["argmax_ids"], want), (lo, hi, g["argmax_ids"][:4], want[:4])
+        if lo < vocab:
+            assert np.isnan(g["log_z"]).all(), (lo, hi)
+
+
 @pytest.mark.parametrize("rows,vocab", [(5, 300), (64, 1000), (130, 1000), (256, 1000)])
 def test_log_z_of_rows_with_inf_blocks(sampler, rows, vocab):
     """Columns of -inf, whole blocks of them too, have no weight in log z; a
