@@ -1267,10 +1267,10 @@ __device__ __attribute__((noinline)) uint32_t nuc_large_group(uint32_t c0, uint3
 }
 
 // The select pass's row finalize: exact decisions over the compacted ranges.
-// Every thread of the workgroup calls it. Returns true (uniformly) when the
-// row has to take the exact path.
+// Every thread of the workgroup calls it. handed: a window row that row_fin
+// handed over. Returns true (uniformly) when the row has to take the exact path.
 template <int G>
-__device__ __forceinline__ bool nuc_select_fin(const SampleArgs& a, uint32_t row) {
+__device__ __forceinline__ bool nuc_select_fin(const SampleArgs& a, uint32_t row, bool handed) {
     NucFinSmem& sm = g_fin;
     const uint32_t tid = tid_x();
     const int lane = lane_id(), wv = (int)(tid / kWave);
@@ -1741,7 +1741,7 @@ __device__ __forceinline__ bool nuc_select_fin(const SampleArgs& a, uint32_t row
             dg.maxl = maxl;
             dg.boundary = last_key != ~0ull ? rank_val(last_key) : maxl;
             // (a window row handed over is an exact fallback to the caller)
-            dg.path = row_mode(P, false, a.vocab) == kModeWindow ? LCS_PATH_GENERAL : LCS_PATH_NUCLEUS;
+            dg.path = handed ? LCS_PATH_GENERAL : LCS_PATH_NUCLEUS;
             dg.sum = SK;
             dg.kept_sum = kept_sum;
             a.diag[row] = dg;
@@ -1925,7 +1925,7 @@ __global__ __launch_bounds__(kFT) void nuc_select_fin_kernel(SampleArgs a) {
     if (!nuc_fin_row(a, row, P, masked)) return;
     NPROF(row, 15);
     const bool exact = (a.nrow[row - a.nuc_row0].flags & kNucFallback) != 0u;
-    if (exact || nuc_select_fin<G>(a, row)) {
+    if (exact || nuc_select_fin<G>(a, row, row_mode(P, masked, a.vocab) == kModeWindow)) {
         stage_args(&sm.l.args, a);
         exact_row<kFT, kFbBins, kFbCap, kFbHistCap, G>(sm.l.args, row, sm.u.ex);
     }

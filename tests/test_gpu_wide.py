@@ -63,6 +63,18 @@ def test_wide_rows(sampler, V, rows, dtype, params):
     assert np.array_equal(h["ids"], g["ids"]) and np.array_equal(h["top_ids"], g["top_ids"])
 
 
+@pytest.mark.parametrize("V,dtype,params", [
+    (50257, "f32", dict(temperature=1.5, min_p=0.02, top_p=0.9)),
+    (9000, "bf16", dict(temperature=0.7, min_p=0.05)),
+])
+def test_constrained_min_p_rows_report_the_nucleus_path(sampler, V, dtype, params):
+    """A min-p row under a mask is the nucleus kernels' own, not one handed over."""
+    w, w32 = make(V, 4, dtype, 79, **params)
+    w.mask = w32.mask = W.pack_mask(np.random.default_rng(V).random((4, V)) < 0.95)
+    o = O.sample_batch(w32, threads=16)
+    compare(w32, sampler.sample(w), o, "constrained", expect_paths={6})
+
+
 def test_wide_rows_beside_others(sampler):
     """Greedy, top-k, narrow and wide min-p, top-p and masked rows in one batch."""
     w, _ = make(40000, 24, "f32", 5, **PEN)
