@@ -1076,6 +1076,16 @@ __global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(1, 2))) void
     const int d1 = min(first_mass(u * K_hi * (1.0 + kGuard)), kb);
     ib[3] = d0;
     ie[3] = d1;
+    // Candidates past the bins have no sub-bins to go by, so a top-k, top-p or
+    // draw decision that may fall among them takes the exact path; min-p's
+    // does not, it counts and sums its range key by key. (A sub-bin that they
+    // share with bins ahead of the last one has too large a mass with them,
+    // which leaves it the first to reach a target inside it.)
+    bool past = false;
+    if (nr->flags & kNucOff) {
+#pragma unroll
+        for (int i = 0; i < 4; ++i) past = past || (i != 2 && ib[i] < NB && ie[i] == NB - 1);
+    }
     // sort the slots by start (a five-exchange network), then merge
     // overlapping or adjacent intervals in order, writing each merged range
     // as it closes
@@ -1119,8 +1129,6 @@ __global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(1, 2))) void
     nr->nr = nm_;
     nr->list_n = 0u;
     NPROF(row, 3);
-    // (a decision among candidates past the bins has no sub-bins to go by)
-    const bool past = (nr->flags & kNucOff) && cur_b < NB && cur_e == NB - 1;
     if (total > kNucList || ncand != ncand_row || past) nr->flags |= kNucFallback;
 }
 

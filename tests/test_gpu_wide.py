@@ -75,6 +75,29 @@ def test_constrained_min_p_rows_report_the_nucleus_path(sampler, V, dtype, param
     compare(w32, sampler.sample(w), o, "constrained", expect_paths={6})
 
 
+@pytest.mark.parametrize("V,dtype,params", [
+    (128256, "f32", dict(temperature=3.0, min_p=1e-6, top_p=1.0, **PEN)),
+    (128256, "f32", dict(temperature=3.0, min_p=1e-6, top_p=0.9, **PEN)),
+    (50257, "bf16", dict(temperature=2.0, min_p=1e-9, top_p=1.0, **PEN)),
+    (50257, "f32", dict(temperature=2.0, min_p=1e-30, top_p=1.0, **PEN)),     # below every outlier
+    (128256, "f32", dict(temperature=1.5, min_p=0.02, top_p=0.9, **PEN)),     # inside the bins
+])
+def test_min_p_cut_past_the_bins(sampler, V, dtype, params):
+    """Constrained rows whose penalised outliers (one id 60 logits down, one 25)
+    lie past the histogram's bins: a min-p cut between them or beyond is no
+    reason for the exact path."""
+    w, w32 = make(V, 8, dtype, 78, **params)
+    bits = np.random.default_rng(V).random((8, V)) < 0.95
+    bits[:, :10] = True
+    w.hist_ids.reshape(8, -1)[:, ::6] = 7
+    w.mask = w32.mask = W.pack_mask(bits)
+    w.u[:] = w32.u[:] = np.linspace(0.02, 0.9, 8)   # (a draw in the last bin is one)
+    assert w32.hist_ids is w.hist_ids
+    o = O.sample_batch(w32, threads=16)
+    g = sampler.sample(w)
+    compare(w32, g, o, "past", expect_paths={6})
+
+
 def test_wide_rows_beside_others(sampler):
     """Greedy, top-k, narrow and wide min-p, top-p and masked rows in one batch."""
     w, _ = make(40000, 24, "f32", 5, **PEN)
