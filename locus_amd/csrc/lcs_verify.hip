@@ -32,21 +32,36 @@ namespace lcs {
 // with the running max moved per group and 256 threads, 17.2 with it moved per
 // round, 13.0 with 512 threads), for many the memory stream (4096 bf16 rows, V
 // 163840: 246 -> 234 us, 5.7 TB/s).
+//
+// A row's last round takes 1, 2, 3, 4 or 6 groups a thread where the row has no
+// more: a short row would spend its time on the terms past its end (2048 bf16
+// rows, us a call with eight / as here: V 1000 12.4 / 9.0, V 5000 13.4 / 10.1;
+// 1024 rows of V 70000 33.9 / 29.6). Forms of their own: the code of the other
+// rounds costs a row without one (20 f32 rows of V 128256 13.2 / 13.5), and the
+// registers of eight groups keep short rows out (4096 bf16 rows of V 5000 16.3 /
+// 14.5).
+constexpr int kRound = 8;
+enum RowForm { kRowRounds, kRowTail, kRowShort };   // rounds of kRound groups; and a shorter last one; that one alone
+template <int G>
+RowForm row_form(uint32_t vocab, uint32_t nt) {
+    const uint32_t ng = (vocab + G - 1u) / G, left = ng % (kRound * nt);
+    return ng <= 4u * nt ? kRowShort : left != 0u && left <= 6u * nt ? kRowTail : kRowRounds;
+}
 struct RowLane {
-    float om;
-    double os;
+    float om, b;
+    double os, corr;
     uint32_t bg;
 };
-template <int G, int NT>
-__device__ __forceinline__ RowLane stream_row(const void* rowp, uint32_t V) {
-    constexpr int U = 8;                   // 16-byte groups in flight per thread
+// Rounds of U groups a thread over groups first .. end of a row of ng.
+template <int G, int NT, int U>
+__device__ __forceinline__ void stream_rounds(const void* rowp, uint32_t V, uint32_t ng, uint32_t first, uint32_t end,
+                                              RowLane& l) {
     constexpr float kL2E = 1.4426950408889634f;
     const float NEG = -__builtin_huge_valf();
-    const uint32_t ng = (V + G - 1) / G;
-    float om = NEG, b = 0.0f;
-    double os = 0.0, corr = 1.0;
-    uint32_t bg = 0xffffffffu;
-    for (uint32_t g0 = 0; g0 < ng; g0 += NT * U) {
+    float om = l.om, b = l.b;
+    double os = l.os, corr = l.corr;
+    uint32_t bg = l.bg;
+    for (uint32_t g0 = first; g0 < end; g0 += NT * U) {
         uint4 r[U];
 #pragma unroll
         for (int u = 0; u < U; ++u) {
@@ -91,7 +106,23 @@ __device__ __forceinline__ RowLane stream_row(const void* rowp, uint32_t V) {
             }
         }
     }
-    return RowLane{om, os, bg};
+    l = RowLane{om, b, os, corr, bg};
+}
+template <int G, int NT, RowForm F>
+__device__ __forceinline__ RowLane stream_row(const void* rowp, uint32_t V) {
+    const uint32_t ng = (V + G - 1) / G;
+    RowLane l{-__builtin_huge_valf(), 0.0f, 0.0, 1.0, 0xffffffffu};
+    const uint32_t end = F == kRowRounds ? ng : F == kRowTail ? ng / (kRound * NT) * (kRound * NT) : 0u;
+    if (F != kRowShort) stream_rounds<G, NT, kRound>(rowp, V, ng, 0u, end, l);
+    if (F != kRowRounds) {   // (uniform branches; row_form leaves no more groups than these take)
+        const uint32_t n = (ng - end + NT - 1u) / NT;
+        if (F == kRowTail && n > 4u) stream_rounds<G, NT, 6>(rowp, V, ng, end, ng, l);
+        else if (n > 3u) stream_rounds<G, NT, 4>(rowp, V, ng, end, ng, l);
+        else if (n > 2u) stream_rounds<G, NT, 3>(rowp, V, ng, end, ng, l);
+        else if (n > 1u) stream_rounds<G, NT, 2>(rowp, V, ng, end, ng, l);
+        else stream_rounds<G, NT, 1>(rowp, V, ng, end, ng, l);
+    }
+    return l;
 }
 
 // The block's max and its first index, and the row's sum of exponentials
@@ -115,7 +146,7 @@ __device__ __forceinline__ double reduce_row(const RowLane& l, const void* rowp,
     return block_sum<NT>(sc, redd);
 }
 
-template <int G, int NT>
+template <int G, int NT, RowForm F>
 __global__ __launch_bounds__(NT) void verify_kernel(VerifyArgs a) {
     __shared__ float redf[NT / kWave];
     __shared__ uint32_t redu[NT / kWave];
@@ -125,7 +156,7 @@ __global__ __launch_bounds__(NT) void verify_kernel(VerifyArgs a) {
     if (row >= rows) return;
     const uint32_t V = a.vocab;
     const void* rowp = static_cast<const char*>(a.logits) + (uint64_t)row * a.row_stride * (16u / G);
-    const RowLane l = stream_row<G, NT>(rowp, V);
+    const RowLane l = stream_row<G, NT, F>(rowp, V);
     float bm;
     uint32_t idx;
     const double z = reduce_row<G, NT>(l, rowp, V, bm, idx, redf, redu, redd);
@@ -150,7 +181,7 @@ __global__ __launch_bounds__(NT) void verify_kernel(VerifyArgs a) {
 // rows of V 128256, top 5: 99.8 us on the sliced path (85 + 18) -> 55.1, 4.8 TB/s.
 constexpr int kLpThreads = 512;
 constexpr uint32_t kLpLanes = 64, kLpCand = 256;   // lanes read again, candidates ranked
-template <int G>
+template <int G, RowForm F>
 __global__ __launch_bounds__(kLpThreads) void logprobs_kernel(LogprobArgs a) {
     constexpr int NT = kLpThreads, NW = NT / kWave;
     __shared__ float redf[NW];
@@ -166,7 +197,7 @@ __global__ __launch_bounds__(kLpThreads) void logprobs_kernel(LogprobArgs a) {
     if (row >= a.rows) return;
     const uint32_t V = a.vocab, ng = (V + G - 1) / G, ntop = a.n_top;
     const void* rowp = static_cast<const char*>(a.logits) + (uint64_t)row * a.row_stride * (16u / G);
-    const RowLane l = stream_row<G, NT>(rowp, V);
+    const RowLane l = stream_row<G, NT, F>(rowp, V);
     lmax[tid] = l.om;
     if (tid == 0) { nl = 0u; nc = 0u; }
     float bm;
@@ -255,9 +286,18 @@ __global__ __launch_bounds__(kLpThreads) void logprobs_kernel(LogprobArgs a) {
     if (wv == 0 && (uint32_t)lane >= have && (uint32_t)lane < ntop) put((uint32_t)lane, ~0ull);
 }
 
+template <int G>
+static void launch_lp(const LogprobArgs& a, hipStream_t st) {
+    const dim3 grid(a.rows), block(kLpThreads);
+    const RowForm f = row_form<G>(a.vocab, kLpThreads);
+    if (f == kRowRounds) hipLaunchKernelGGL((logprobs_kernel<G, kRowRounds>), grid, block, 0, st, a);
+    else if (f == kRowTail) hipLaunchKernelGGL((logprobs_kernel<G, kRowTail>), grid, block, 0, st, a);
+    else hipLaunchKernelGGL((logprobs_kernel<G, kRowShort>), grid, block, 0, st, a);
+}
+
 hipError_t launch_logprobs(const LogprobArgs& a, uint32_t dtype, hipStream_t st) {
-    if (dtype == LCS_BF16) hipLaunchKernelGGL(logprobs_kernel<8>, dim3(a.rows), dim3(kLpThreads), 0, st, a);
-    else hipLaunchKernelGGL(logprobs_kernel<4>, dim3(a.rows), dim3(kLpThreads), 0, st, a);
+    if (dtype == LCS_BF16) launch_lp<8>(a, st);
+    else launch_lp<4>(a, st);
     return hipGetLastError();
 }
 
@@ -275,19 +315,33 @@ __global__ __launch_bounds__(kAcceptSeqs * kWave) void accept_kernel(VerifyArgs 
     if (lane == 0u) a.accept_len[seq] = acc;
 }
 
-// Threads per row: a row of more than two rounds of 512 threads takes 512 (us
-// a call with 256 / 512 / 1024 threads, f32, V 128256: 20 rows 17.2 / 13.0 /
-// 13.0, 128 rows 19.6 / 15.6 / 17.2, 2048 rows 187.5 / 187.1 / 189; bf16, V
-// 163840, 4096 rows 238.3 / 233.8 / 267), except where about two rows a CU
-// make one uneven round of the larger workgroups (512 rows: 51.4 / 52.7, bf16
-// 34.9 / 36.6). A shorter row leaves them idle (2048 rows of V 5000: 13.3 /
-// 17.1).
+template <int G, int NT>
+static void launch_nt(const VerifyArgs& a, uint32_t rows, hipStream_t st) {
+    const RowForm f = row_form<G>(a.vocab, NT);
+    if constexpr (NT == 256) {   // (512 threads take long rows only)
+        if (f == kRowShort) {
+            hipLaunchKernelGGL((verify_kernel<G, NT, kRowShort>), dim3(rows), dim3(NT), 0, st, a);
+            return;
+        }
+    }
+    if (f == kRowRounds) hipLaunchKernelGGL((verify_kernel<G, NT, kRowRounds>), dim3(rows), dim3(NT), 0, st, a);
+    else hipLaunchKernelGGL((verify_kernel<G, NT, kRowTail>), dim3(rows), dim3(NT), 0, st, a);
+}
+
+// Threads per row (us a call with 256 / 512 threads). Up to a row a CU, a row
+// of more than two rounds of 512 threads takes 512: f32, V 128256, 16 rows 14.3
+// / 12.3, 128 rows 19.0 / 15.2, 200 rows 20.2 / 19.9 (256 rows 23.2 / 24.1);
+// bf16, V 128256, 128 rows 14.9 / 12.7, 256 rows 16.9 / 15.4, V 70000, 16 rows
+// 9.4 / 9.0. Above, smaller workgroups even the CUs out (f32, V 128256, 300 rows
+// 27.9 / 32.9, 512 rows 42.7 / 45.2; bf16, V 163840, 300 rows 23.5 / 26.2, 1024
+// rows 59.3 / 60.7; 2048 rows of V 5000 10.1 / 16.7), except for thousands of
+// long bf16 rows (V 163840, 1536 rows 93.1 / 90.7, 4096 rows 229.7 / 228.8).
 template <int G>
 static void launch_rows(const VerifyArgs& a, hipStream_t st) {
-    const uint32_t rows = a.n_seq * a.rows_per_seq;
-    const bool wide = (a.vocab + G - 1u) / G > 8192u && (rows <= 256u || rows > 768u);
-    if (wide) hipLaunchKernelGGL((verify_kernel<G, 512>), dim3(rows), dim3(512), 0, st, a);
-    else hipLaunchKernelGGL((verify_kernel<G, 256>), dim3(rows), dim3(256), 0, st, a);
+    const uint32_t rows = a.n_seq * a.rows_per_seq, ng = (a.vocab + G - 1u) / G;
+    const bool wide = ng > 8192u && (rows <= 256u || (G == 8 && rows > 1024u && ng > 16384u));
+    if (wide) launch_nt<G, 512>(a, rows, st);
+    else launch_nt<G, 256>(a, rows, st);
 }
 
 hipError_t launch_verify(const VerifyArgs& a, hipStream_t st) {

@@ -72,3 +72,29 @@ def test_rows_in_one_workgroup(sampler, V, rows, dtype, n_top):
     sampler.sample_dev(d, o2, lp_ids=torch.from_numpy(chosen).cuda())
     torch.cuda.synchronize()
     assert torch.equal(o["top_ids"], o2["top_ids"]) and torch.equal(o["ids"], o2["ids"])
+
+
+@pytest.mark.parametrize("dtype", ["f32", "bf16"])
+@pytest.mark.parametrize("NT,before", [(256, 0), (512, 8192)])   # threads per row, groups ahead of the last round
+def test_verify_rows_that_end_in_any_slot_of_a_round(sampler, NT, before, dtype):
+    """A row's last round takes 1, 2, 3, 4, 6 or 8 groups of 16 bytes a thread:
+    rows that end with the first and the last group of each, the maximum among
+    the row's last ids, against float64."""
+    G, rows = 8 if dtype == "bf16" else 4, 4
+    for k in range(8):
+        for V in ((before + k * NT) * G + 1, (before + (k + 1) * NT) * G - 1, (before + (k + 1) * NT) * G):
+            g = np.random.default_rng([V, NT])
+            x = (g.standard_normal((rows, V), dtype=np.float32) * 2).astype(np.float32)
+            x[0, V - 1] = x[1, V // 2] = x[1, V - 1] = 30.0
+            logits = W.bf16_rne(x) if dtype == "bf16" else x
+            f = (W.bf16_to_f32(logits) if dtype == "bf16" else x).astype(np.float64)
+            draft = np.array([V - 1, V // 2, 0, V - 1], np.int32)
+            w = W.Workload("rounds", rows, V, dtype, logits, None, None, None, n_seq=2, rows_per_seq=2, draft=draft)
+            got = sampler.verify(w)
+            am = f.argmax(1)
+            m = f.max(1, keepdims=True)
+            lp = f[np.arange(rows), draft] - (m + np.log(np.exp(f - m).sum(1, keepdims=True)))[:, 0]
+            assert np.array_equal(got["argmax_ids"], am), (V, got["argmax_ids"], am)
+            assert (np.abs(got["draft_lp"] - lp) <= 1e-5).all(), (V, got["draft_lp"], lp)
+            hit = (am == draft).reshape(2, 2)
+            assert got["accept_len"].tolist() == [int(h[0]) + int(h[0] and h[1]) for h in hit]
