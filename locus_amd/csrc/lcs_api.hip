@@ -211,15 +211,19 @@ __global__ void clear_words(uint32_t* w, uint32_t n) {
 
 // Whether a batch with logprobs is greedy rows without penalties or a mask
 // (lcs_logprobs, or lcs_sample as such) that the one-kernel path serves: a
-// workgroup per row streams it once. Below 64 rows a long row is faster cut
-// into slices (us, sliced / whole: V 128256 bf16, 16 rows 11.2 / 12.0, 64 rows
-// 13.9 / 12.5, 1024 rows 99.8 / 55.1; f32 11.0 / 12.7, 14.8 / 14.5, 113.6 /
-// 101.1); up to 8192 16-byte groups the second launch costs more than the
-// slices save (V 32000, 16 rows 11.1 / 7.7).
+// workgroup per row streams it once. Up to 8192 16-byte groups a second launch
+// costs more than slices save (us, sliced / whole: V 32000, 16 rows 11.1 / 7.8,
+// 1024 rows 41.3 / 27.6). A few longer rows are faster cut into slices, as long
+// as these run in one go: f32, V 128256, 16 rows 11.0 / 12.7, 64 rows 12.9 /
+// 14.1, 65 rows 15.6 / 14.2, V 262144, 72 rows 22.3 / 23.0, 80 rows 24.0 /
+// 23.1; bf16, V 128256, 16 rows 11.2 / 12.0, 64 rows 12.8 / 12.1, V 262144, 64
+// rows 18.3 / 18.7, 65 rows 20.6 / 20.0; f32, V 100000, 64 rows 12.6 / 11.3.
 bool plain_greedy(const lcs_batch* b, const lcs_out* o) {
     if (!b->params_host || b->mask || b->raw_stats || o->diag || b->win_slot || (b->flags & LCS_WRITE_PENALIZED)) return false;
     const uint32_t g = b->dtype == LCS_BF16 ? 8u : 4u;
-    if (b->rows < 64u && (b->vocab + g - 1u) / g > 8192u) return false;
+    const uint32_t ng = (b->vocab + g - 1u) / g;
+    const uint32_t sliced = ng <= 8192u ? 0u : ng <= 28672u ? 63u : ng <= 49152u ? 64u : 72u;   // rows up to which slices win
+    if (b->rows <= sliced) return false;
     for (uint32_t r = 0; r < b->rows; ++r) {
         const lcs_params& p = b->params_host[r];
         const bool pen = !(p.repeat_penalty == 1.0f && p.frequency_penalty == 0.0f && p.presence_penalty == 0.0f);
