@@ -1064,7 +1064,12 @@ __global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(1, 2))) void
         const float xm = (float)log((double)P.min_p);
         const float d = 1e-4f * fmaxf(1.0f, fabsf(xm));
         const int b0 = (int)nuc_bin(nuc_f(xm + d, sx)), b1 = (int)nuc_bin(nuc_f(xm - d, sx));
-        ib[2] = b0;
+        // The last survivor's key is wanted too, and in a confident row no
+        // candidate between the cut's bin edge and the cut may be one: the
+        // range starts at the last bin ahead of it that holds candidates (64
+        // rows of V 32000, a few ids 12 logits up: 184 us a call, one row in
+        // 16 on the exact path, -> 79).
+        ib[2] = cb(b0) > 0u ? first_count(cb(b0)) : b0;
         ie[2] = b1;
         km_lo = min(max(1u, cb(b0)), K);
         km_hi = min(max(1u, hc[b1]), K);

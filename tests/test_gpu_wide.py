@@ -98,6 +98,29 @@ def test_min_p_cut_past_the_bins(sampler, V, dtype, params):
     compare(w32, g, o, "past", expect_paths={6})
 
 
+@pytest.mark.parametrize("V,dtype,params", [
+    (32000, "f32", dict(temperature=1.5, min_p=0.01, top_p=0.9)),
+    (32000, "bf16", dict(temperature=1.5, min_p=0.01, **PEN)),
+    (128256, "f32", dict(temperature=0.8, min_p=0.05, top_p=0.95, **PEN)),
+    (700, "f32", dict(temperature=1.0, min_p=0.1, top_k=600)),
+])
+def test_min_p_cut_in_an_empty_bin(sampler, V, dtype, params):
+    """Constrained confident rows (eight ids far above the rest): no candidate
+    in the min-p cut's own bin survives, which is no reason for the exact path."""
+    rows = 16
+    w, w32 = make(V, rows, "f32", 80, **params)
+    g = np.random.default_rng(V)
+    x = w.logits
+    for r in range(rows):
+        x[r, g.choice(np.arange(10, V), 8, replace=False)] += np.float32(12.0)
+    if dtype == "bf16":
+        w.dtype, w.logits = "bf16", W.bf16_rne(x)
+        w32.logits = W.bf16_to_f32(w.logits)
+    w.mask = w32.mask = W.pack_mask(g.random((rows, V)) < 0.95)
+    o = O.sample_batch(w32, threads=16)
+    compare(w32, sampler.sample(w), o, "empty bin", expect_paths={6})
+
+
 def test_wide_rows_beside_others(sampler):
     """Greedy, top-k, narrow and wide min-p, top-p and masked rows in one batch."""
     w, _ = make(40000, 24, "f32", 5, **PEN)
