@@ -149,6 +149,35 @@ def test_row_tiles_are_exact(sampler, rows, vocab, hidden):
         assert np.array_equal(h[k], g[k]) and np.array_equal(out[k].cpu().numpy(), g[k]), k
 
 
+# One or two cases per tile of lmhead_tile (rows, vocab, the tile's 64-column and
+# row counts, k-steps a stage holds, stages of its ring), each run over more
+# stages than the ring has; tests/test_lmhead_shape.py holds the choice of the
+# tile to this list. 256 CUs.
+STEADY = [
+    (3, 300, 1, 64, 2, 6), (64, 20001, 2, 64, 2, 4), (64, 33001, 4, 64, 2, 4), (2, 80001, 5, 64, 2, 3),
+    (17, 100001, 4, 64, 4, 2), (128, 257, 2, 128, 2, 4), (300, 1001, 2, 128, 2, 4), (128, 33001, 4, 128, 2, 3),
+    (300, 50001, 4, 128, 2, 3), (255, 513, 2, 256, 2, 3), (512, 513, 2, 256, 2, 3), (256, 33001, 4, 256, 4, 2),
+    (511, 50257, 4, 256, 4, 2)]
+
+
+@pytest.mark.parametrize("hidden", [320, 384, 512])   # 5, 6 and 8 stages of 64 k, twice as many of 32
+@pytest.mark.parametrize("rows,vocab", [c[:2] for c in STEADY])
+def test_stages_past_the_ring_are_exact(sampler, rows, vocab, hidden):
+    torch = sampler.torch
+    say("stages", rows, vocab, hidden)
+    rng = np.random.default_rng([rows, vocab, hidden])
+    xi = rng.integers(-4, 5, (rows, hidden)).astype(np.float32)
+    wi = rng.integers(-3, 4, (vocab, hidden)).astype(np.float32)
+    # (float64 holds these integer sums exactly; on the device, where it is quick)
+    x, w = torch.from_numpy(xi).cuda(), torch.from_numpy(wi).cuda()
+    ref = (x.double() @ w.double().t()).float().cpu().numpy()
+    cols = rng.choice(vocab, min(vocab, 500), replace=False)
+    assert np.array_equal(ref[:, cols], xi.astype(np.float64) @ wi[cols].T.astype(np.float64))
+    g = run(sampler, x.to(torch.bfloat16), w.to(torch.bfloat16))
+    assert np.array_equal(g["logits"], ref)
+    check_epilogue(g)
+
+
 @pytest.mark.parametrize("rows,vocab", [(3, 1), (5, 70), (64, 300), (130, 513)])
 def test_argmax_stays_in_range_for_nan_and_inf(sampler, rows, vocab):
     """Rows of NaN, of -inf and with one +inf: the argmax is an id of the
