@@ -123,7 +123,7 @@ typedef struct lcs_row_diag {
     float maxl;         /* max penalised candidate logit */
     float boundary;     /* logit of the last survivor */
     uint32_t path;      /* implementation path taken (LCS_PATH_*) */
-    uint32_t reserved;
+    uint32_t reserved;  /* 1: a window row that the nucleus kernels decided, else 0 */
     double sum;         /* softmax normaliser over the candidate list */
     double kept_sum;    /* mass of the survivors */
 } lcs_row_diag;

@@ -1755,6 +1755,7 @@ __device__ __forceinline__ bool nuc_select_fin(const SampleArgs& a, uint32_t row
             dg.boundary = last_key != ~0ull ? rank_val(last_key) : maxl;
             // (a window row handed over is an exact fallback to the caller)
             dg.path = handed ? LCS_PATH_GENERAL : LCS_PATH_NUCLEUS;
+            dg.reserved = handed ? 1u : 0u;
             dg.sum = SK;
             dg.kept_sum = kept_sum;
             a.diag[row] = dg;

@@ -58,7 +58,10 @@ def test_wide_rows(sampler, V, rows, dtype, params):
     w, w32 = make(V, rows, dtype, 77, **params)
     o = O.sample_batch(w32, threads=16)
     g = sampler.sample(w)
-    compare(w32, g, o, "wide", expect_paths={2, 3, 4} if params.get("min_p") else {4, 6})
+    # (min-p rows: handed over and decided there; the others: in the bins, their
+    # outliers summed apart, not on the exact path)
+    compare(w32, g, o, "wide", expect_paths={4} if params.get("min_p") else {6})
+    assert (g["diag"]["reserved"] == (1 if params.get("min_p") else 0)).all(), g["diag"]["reserved"].tolist()
     h = sampler.sample(w, use_host_params=False)   # modes unknown to the host: every kernel is launched
     assert np.array_equal(h["ids"], g["ids"]) and np.array_equal(h["top_ids"], g["top_ids"])
 
@@ -136,6 +139,7 @@ def test_wide_rows_beside_others(sampler):
     o = O.sample_batch(w, threads=16, has_mask=has)
     g = sampler.sample(w, has_mask=sampler.torch.from_numpy(has).cuda())
     compare(w, g, o, "beside")
+    assert g["diag"]["reserved"].tolist() == [0] * 12 + [1] * 4 + [0] * 8
     path = g["diag"]["path"].tolist()
     assert set(path[:4]) == {1} and set(path[4:8]) == {5} and set(path[8:12]) <= {2, 3} and set(path[12:16]) == {4}, path
 
