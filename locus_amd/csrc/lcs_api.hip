@@ -236,10 +236,23 @@ bool plain_greedy(const lcs_batch* b, const lcs_out* o) {
 // T ln(1 / min_p) logits below the maximum (T 0.7, min-p 0.05: 2.1; T 1, 0.01:
 // 4.6; T 1.5, 0.05: 4.5). With logits of spread 2 to 3, a cut 4 below the
 // maximum of V 128256 leaves more than the 64 ids a slice's record holds. One
-// row that overflows costs the call 450-500 us in row_fin's exact path, the
-// five nucleus launches 9-10 us where no row does (V 128256, us a call without
-// / with them: flat rows, 1 row 516 / 84, 64 rows 544 / 117; confident rows, 1
-// row 16.0 / 25.2, 64 rows 22.5 / 32.9).
+// row that overflows costs the call 70-550 us in row_fin's exact path, by V; the
+// five nucleus launches cost 9-12 us where no row does, which the host cannot
+// know. Us a call without / with them (f32, 512-id histories; spread 2, spread 3
+// and confident: spread 2 with eight ids 12 above):
+//                        spread 2     spread 3     confident
+//   T 1, min-p 0.01
+//     V 8000,    1 row    88 /  70     71 /  71     15 / 27
+//     V 8000,   64 rows  117 /  83     95 /  82     16 / 27
+//     V 32000,   1 row   113 /  70     20 /  30     15 / 27
+//     V 32000,  64 rows  247 /  84    144 /  87     26 / 35
+//     V 128256,  1 row   287 /  74    253 /  71     26 / 34
+//     V 128256, 64 rows  563 / 106    300 / 104    267 / 87
+//   T 1.5, min-p 0.01
+//     V 32000,   1 row   242 /  70    114 /  70     22 / 31
+//     V 128256, 64 rows  652 / 110    564 / 106    286 / 101
+// At T 1, min-p 0.02 (3.9) the same rows take 81 to 561 us (confident ones 14
+// to 30) without them: the line lies where the settings meet overflows often.
 constexpr float kWideWindow = 4.0f;
 bool wide_windows(const lcs_batch* b) {
     for (uint32_t r = 0; r < b->rows; ++r) {

@@ -65,8 +65,8 @@ constexpr int kGenThreads = 1024;
 constexpr uint32_t kGenBins = 2048;
 constexpr uint32_t kGenCap = 2048;
 constexpr uint32_t kGenHistCap = 8192;
-// inline fallback inside the nucleus finalize kernels (256 threads; the
-// LDS block shares the nucleus passes' union, so it stays within 32 KB)
+// inline fallback inside the nucleus select finalize (512 threads, an LDS block
+// of the finalize's own)
 constexpr uint32_t kFbBins = 512;
 constexpr uint32_t kFbCap = 512;
 constexpr uint32_t kFbHistCap = kFastHistMax;

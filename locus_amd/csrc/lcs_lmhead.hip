@@ -109,7 +109,7 @@ __device__ __forceinline__ void block_sync() {
 // row tiles share x through the L2 by running in step (1024 rows: 1013 against
 // 1057 us with a start of its own).
 template <int VT, int BR, int ST, int NW = 4, int KS = 2, bool BIG = false>
-__global__ __launch_bounds__(NW * kWave, NW == 8 ? 2 : VT * BR == 1024 ? 1 : 2) void lmhead_tile(LmArgs a) {
+__global__ __launch_bounds__(NW * kWave, 2) void lmhead_tile(LmArgs a) {
     constexpr uint32_t kTV = 64u * VT;        // columns per workgroup
     constexpr int kTK = 16 * KS;              // k per LDS stage
     constexpr uint32_t kTRowB = kTK * 2;      // bytes of a row in a stage

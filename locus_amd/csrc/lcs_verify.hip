@@ -36,10 +36,10 @@ namespace lcs {
 // A row's last round takes 1, 2, 3, 4 or 6 groups a thread where the row has no
 // more: a short row would spend its time on the terms past its end (2048 bf16
 // rows, us a call with eight / as here: V 1000 12.4 / 9.0, V 5000 13.4 / 10.1;
-// 1024 rows of V 70000 33.9 / 29.6). Forms of their own: the code of the other
-// rounds costs a row without one (20 f32 rows of V 128256 13.2 / 13.5), and the
-// registers of eight groups keep short rows out (4096 bf16 rows of V 5000 16.3 /
-// 14.5).
+// 1024 rows of V 70000 33.9 / 29.6). Forms of their own: a row without a short
+// round keeps its plain loop (the short ones beside it moved 20 f32 rows of V
+// 128256 from 13.2 to 13.5), and the registers of eight groups keep short rows
+// out (4096 bf16 rows of V 5000 16.3 / 14.5).
 constexpr int kRound = 8;
 enum RowForm { kRowRounds, kRowTail, kRowShort };   // rounds of kRound groups; and a shorter last one; that one alone
 template <int G>
