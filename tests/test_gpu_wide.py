@@ -83,6 +83,7 @@ def test_constrained_min_p_rows_report_the_nucleus_path(sampler, V, dtype, param
     (128256, "f32", dict(temperature=3.0, min_p=1e-6, top_p=0.9, **PEN)),
     (50257, "bf16", dict(temperature=2.0, min_p=1e-9, top_p=1.0, **PEN)),
     (50257, "f32", dict(temperature=2.0, min_p=1e-30, top_p=1.0, **PEN)),     # below every outlier
+    (128256, "f32", dict(temperature=3.0, min_p=0.01, top_p=1.0, **PEN)),     # between the bins' end and the outliers
     (128256, "f32", dict(temperature=1.5, min_p=0.02, top_p=0.9, **PEN)),     # inside the bins
 ])
 def test_min_p_cut_past_the_bins(sampler, V, dtype, params):
